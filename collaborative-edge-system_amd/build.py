@@ -58,6 +58,7 @@ FILE_FLAGS = {
     # the projection's epilogue rounds like the reference's separate ops (see layers.hip);
     # M0 is set by the LDS-DMA assembly
     "gemm.hip": ["-ffp-contract=off", "-Wno-inline-asm"],
+    "gemm_skinny.hip": ["-ffp-contract=off", "-Wno-inline-asm"],
 }
 
 

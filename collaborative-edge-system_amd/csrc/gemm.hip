@@ -39,31 +39,11 @@
 // (f64 for f64 tensors).
 #include <type_traits>
 
-#include "cea_kernels.hpp"
 #include "cea_lds_dma.hpp"
+#include "gemm_common.hpp"
 
 namespace cea {
 namespace {
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-template <typename T> struct GMfma;
-template <> struct GMfma<bf16> {
-  typedef bf16x8 frag;
-  static __device__ __forceinline__ f32x4 run(frag a, frag b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-  }
-};
-template <> struct GMfma<f16> {
-  typedef f16x8 frag;
-  static __device__ __forceinline__ f32x4 run(frag a, frag b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
-  }
-};
-
-enum { kPlain = 0, kGated = 1 };
 
 constexpr int G_THREADS = 512;                       // 8 waves, two per SIMD
 constexpr int G_BM = 256;                            // tokens per tile
@@ -75,30 +55,8 @@ constexpr int G_OPER = G_BM * G_ROW;                 // 32 KB per operand per sl
 constexpr int G_STAGE = 2 * G_OPER;                  // weight slice, then token slice
 constexpr int G_LDS = G_NST * G_STAGE;               // 128 KB
 constexpr int G_LOADS = G_OPER / (G_THREADS * 16);   // 16-byte loads per lane per operand
-constexpr uint32_t kOutOfRange = 0x80000000u;        // above every resource's range
 constexpr int kLgkm0 = 0xC07F;   // s_waitcnt lgkmcnt(0), vmcnt / expcnt left at their maximum
 static_assert(G_LOADS == 4 && G_BM == G_BW, "the load pattern assumes 4 x 8 rows per wave");
-
-struct GemmParams {
-  const void* x;    // [M, K], row stride ldx
-  const void* wg;   // [N, K], row stride ldw (gated: the gate rows)
-  const void* wu;   // gated: the up rows, same row stride
-  const void* bg;   // [N] or null (gated: gate bias)
-  const void* bu;   // gated: up bias or null
-  void* y;          // [M, N], row stride ldy
-  int64_t ldx, ldw, ldy;
-  int32_t M, N, K;  // N = output columns
-  int32_t tiles_m, tiles_n, group_m;
-  int32_t vec_out;  // 2: 16-byte row chunks, 1: 4-element stores, 0: element stores
-};
-
-// 16-byte group swizzle of a slice row (8 groups of 16 bytes): group c of row r sits at group
-// c ^ g_swz(r).  A fragment read has 16 rows per 16-lane quarter and the quarters read groups
-// c, c+1, c+2, c+3.  Measured on gfx950 (LDS bank-conflict counter), the reads behave as if 32
-// lanes share a 512-byte bank window; this swizzle gives distinct 16-byte slots for any 32
-// lanes (rows of equal r & 3 in one window), for any 16 lanes within 256 bytes and for any 8
-// within 128 bytes.  Depends on r & 15 only.
-__device__ __forceinline__ int g_swz(int r) { return ((r >> 1) & 7) ^ ((r & 1) << 2); }
 
 // Tile (token block, weight block) of this workgroup.
 __device__ __forceinline__ void tile_of(const GemmParams& p, int& tm, int& tn) {
@@ -112,69 +70,6 @@ __device__ __forceinline__ void tile_of(const GemmParams& p, int& tm, int& tn) {
   const int r = b - grp * per_group;
   tm = first + r % gm;
   tn = r / gm;
-}
-
-template <typename T, typename A> __device__ __forceinline__ A rnd_acc(A v) {
-  if constexpr (sizeof(T) >= sizeof(A)) return v;
-  else return (A)round_to<T>((float)v);
-}
-
-// Bias of 4 consecutive columns (zero without a bias, or past n).
-template <typename T, typename A>
-__device__ __forceinline__ void bias4(const void* b, int col, int n, bool vec, A (&v)[4]) {
-  const T* bp = (const T*)b;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) v[j] = A(0);
-  if (bp == nullptr) return;
-  if (vec && col + 3 < n) {
-    T t[4];
-    __builtin_memcpy(t, bp + col, sizeof(t));
-#pragma unroll
-    for (int j = 0; j < 4; ++j) v[j] = (A)to_f32<T>(t[j]);
-  } else {
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (col + j < n) v[j] = load_acc<T, A>(bp + col + j);
-  }
-}
-
-// Stores 4 consecutive columns of one output row.
-template <typename T, typename A>
-__device__ __forceinline__ void store4(T* row, int col, int n, bool vec, const A (&v)[4]) {
-  T t[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) t[j] = store_cast<T, A>(v[j]);
-  if (vec && col + 3 < n) {
-    if constexpr (sizeof(T) == 2) {
-      uint2 raw;
-      __builtin_memcpy(&raw, t, 8);
-      *(uint2*)(row + col) = raw;
-    } else {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) row[col + j] = t[j];
-    }
-  } else {
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (col + j < n) row[col + j] = t[j];
-  }
-}
-
-// The epilogue of 4 consecutive columns: plain y = acc + bias; gated
-// y = T(act(T(gate + b_g))) * T(up + b_u).
-template <typename T, int MODE, int ACT, bool BIAS, typename A>
-__device__ __forceinline__ void finish4(const A (&g)[4], const A (&u)[4], const A (&bg)[4],
-                                        const A (&bu)[4], A (&v)[4]) {
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    if constexpr (MODE == kPlain) {
-      v[j] = BIAS ? add_rn(g[j], bg[j]) : g[j];
-    } else {
-      const A gate = rnd_acc<T, A>(BIAS ? add_rn(g[j], bg[j]) : g[j]);
-      const A up = rnd_acc<T, A>(BIAS ? add_rn(u[j], bu[j]) : u[j]);
-      v[j] = mul_rn(rnd_acc<T, A>(gate_act<ACT, A>(gate)), up);
-    }
-  }
 }
 
 template <typename T, int MODE, int ACT>
@@ -557,6 +452,7 @@ int launch_linear(const cea_tensor* x, const cea_tensor* wg, const cea_tensor* w
   p.vec_out = v16 ? 2 : v8 ? 1 : 0;
   if (p.M == 0 || p.N == 0) return CEA_OK;
   const bool mfma = mfma_path(p, x->dtype, mode);
+  if (mfma && p.M <= kSkinnyTokens) return launch_linear_skinny(p, x->dtype, mode, act, st);
   switch (x->dtype) {
     case CEA_BF16: return launch_typed<bf16>(p, mode, act, mfma, st);
     case CEA_F16: return launch_typed<f16>(p, mode, act, mfma, st);

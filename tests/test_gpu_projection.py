@@ -269,3 +269,31 @@ def test_fused_qkv_projection_views_feed_the_kernels(cea, dev):
     torch.cuda.synchronize()
     assert torch.equal(out, ref)
     assert torch.equal(dout, dref) and torch.equal(dlse, dlref)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,k,n", [
+    (1, 8, 16),        # one K group: seven of the eight waves have no slice
+    (16, 520, 15),     # a full token block; N past a weight block's last full row, element stores
+    (17, 72, 40),      # second token block with one row, a K tail in the second slice
+    (33, 1032, 4100),  # third token block, more weight blocks than compute units
+    (64, 1024, 8200),  # largest token count of the few-token kernel, four blocks per workgroup
+    (65, 136, 24),     # first token count past it
+])
+def test_linear_few_tokens(cea, dev, dtype, m, k, n):
+    """The few-token kernel at the edges of its token blocks, weight blocks and K slices,
+    plain (strided x and output rows) and gated."""
+    g = torch.Generator().manual_seed(m + 3 * k + n)
+    x, w, b = _operands(g, m, k, 2 * n, dtype)
+    xd = torch.zeros(m, k + 8, dtype=dtype, device=dev)[:, :k]
+    xd.copy_(x)
+    wd, bd = w.to(dev), b.to(dev)
+    out = torch.full((m, 2 * n + 16), 7.0, dtype=dtype, device=dev)
+    cea.projection.linear(xd, wd, bd, out=out[:, 8:8 + 2 * n])
+    torch.cuda.synchronize()
+    _check_linear(out[:, 8:8 + 2 * n], x, w, b, f"few tokens {m}x{k}x{n} {dtype}")
+    assert bool((out[:, :8] == 7).all()) and bool((out[:, 8 + 2 * n:] == 7).all())
+    y = cea.projection.linear_gated(xd, wd[:n], wd[n:], bd[:n], bd[n:], "silu")
+    chain = cea.layers.gated_mul(out[:, 8:8 + n].contiguous(), out[:, 8 + n:8 + 2 * n].contiguous(), "silu")
+    torch.cuda.synchronize()
+    _same_as_chain(y, chain, f"few tokens gated {m}x{k}x{n} {dtype}")
