@@ -116,6 +116,15 @@ _SIGNATURES = {
     "cea_gated_mul": (ctypes.c_int, [_P, _P, _P, ctypes.c_int32, ctypes.c_void_p]),
     "cea_linear": (ctypes.c_int, [_P, _P, _P, _P, ctypes.c_void_p]),
     "cea_linear_gated": (ctypes.c_int, [_P, _P, _P, _P, _P, _P, ctypes.c_int32, ctypes.c_void_p]),
+    "cea_linear_workspace_bytes": (
+        ctypes.c_size_t,
+        [ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, ctypes.c_int32, ctypes.c_int32],
+    ),
+    "cea_linear_ws": (ctypes.c_int, [_P, _P, _P, _P, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]),
+    "cea_linear_gated_ws": (
+        ctypes.c_int,
+        [_P, _P, _P, _P, _P, _P, ctypes.c_int32, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p],
+    ),
     "cea_kv_append": (
         ctypes.c_int,
         [_P, _P, _P, _P, _P, _P, _P, _P, ctypes.c_int64, ctypes.c_void_p],

@@ -1217,19 +1217,36 @@ static int check_linear_io(const char* what, const cea_tensor* x, const cea_tens
   return CEA_OK;
 }
 
+size_t cea_linear_workspace_bytes(int64_t M, int64_t N, int64_t K, int32_t dtype, int32_t gated) {
+  if (M <= 0 || N <= 0 || K <= 0) return 0;
+  return linear_workspace_bytes(M, N, K, dtype, gated ? 1 : 0);
+}
+
 int cea_linear(const cea_tensor* x, const cea_tensor* weight, const cea_tensor* bias,
                cea_tensor* y, void* stream) {
+  return cea_linear_ws(x, weight, bias, y, nullptr, 0, stream);
+}
+
+int cea_linear_ws(const cea_tensor* x, const cea_tensor* weight, const cea_tensor* bias,
+                  cea_tensor* y, void* workspace, size_t workspace_bytes, void* stream) {
   int rc;
   CEA_REQUIRE(x != nullptr && weight != nullptr, CEA_EINVAL, "linear: missing tensor");
   if ((rc = check_tensor(weight, "weight", 2, -1, true))) return rc;
   if ((rc = check_linear_io("linear", x, y, weight->size[0]))) return rc;
   if ((rc = check_projection("linear", x, weight, bias, "weight", "bias"))) return rc;
-  return launch_linear(x, weight, nullptr, bias, nullptr, y, 0, 0, (hipStream_t)stream);
+  return launch_linear(x, weight, nullptr, bias, nullptr, y, 0, 0, workspace, workspace_bytes,
+                       (hipStream_t)stream);
 }
 
 int cea_linear_gated(const cea_tensor* x, const cea_tensor* w_gate, const cea_tensor* w_up,
                      const cea_tensor* b_gate, const cea_tensor* b_up, cea_tensor* y,
                      int32_t act, void* stream) {
+  return cea_linear_gated_ws(x, w_gate, w_up, b_gate, b_up, y, act, nullptr, 0, stream);
+}
+
+int cea_linear_gated_ws(const cea_tensor* x, const cea_tensor* w_gate, const cea_tensor* w_up,
+                        const cea_tensor* b_gate, const cea_tensor* b_up, cea_tensor* y,
+                        int32_t act, void* workspace, size_t workspace_bytes, void* stream) {
   int rc;
   CEA_REQUIRE(x != nullptr && w_gate != nullptr && w_up != nullptr, CEA_EINVAL,
               "linear_gated: missing tensor");
@@ -1245,7 +1262,8 @@ int cea_linear_gated(const cea_tensor* x, const cea_tensor* w_gate, const cea_te
               "linear_gated: give both biases or neither");
   CEA_REQUIRE(act >= CEA_ACT_SILU && act <= CEA_ACT_RELU, CEA_EUNSUPPORTED,
               "linear_gated: unknown activation %d", (int)act);
-  return launch_linear(x, w_gate, w_up, b_gate, b_up, y, 1, act, (hipStream_t)stream);
+  return launch_linear(x, w_gate, w_up, b_gate, b_up, y, 1, act, workspace, workspace_bytes,
+                       (hipStream_t)stream);
 }
 
 }  // extern "C"

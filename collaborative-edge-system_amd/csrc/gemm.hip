@@ -11,17 +11,18 @@
 //          [M, 2I] gate/up intermediate never reaches memory.
 //
 // Matrix-core kernel (bf16 / f16, 16-byte aligned rows, K a multiple of 8):
-//   * one workgroup = 8 waves, two per SIMD (256 registers each), computes 256 tokens x 256
-//     weight rows; each wave owns 128 tokens x 64 weight rows, 32 accumulators of
-//     v_mfma_f32_16x16x32 (128 registers); with two waves per SIMD one wave's stalls (load
-//     issue, barrier, the activation epilogue's transcendental latencies) leave the matrix
-//     core to the other;
+//   * one workgroup = 8 waves, two per SIMD (256 registers each), computes 256 tokens (160 or
+//     128 where those pad or quantise less: plan_tiles) x 256 weight rows; each wave owns 128
+//     tokens x 64 weight rows, 32 accumulators of v_mfma_f32_16x16x32 (128 registers); with
+//     two waves per SIMD one wave's stalls (load issue, barrier, the activation epilogue's
+//     transcendental latencies) leave the matrix core to the other;
 //   * the MFMA's A operand is the weight (16 rows) and B the tokens (16 columns), so the 4
 //     accumulator values of a lane are 4 consecutive output features of one token;
 //   * 64-wide K slices of both operands go global -> LDS directly (buffer_load ... lds) into
-//     two stages; a slice row is one 128-byte cache line, so each load instruction touches 8
-//     lines (the address unit's cost is per line touched); rows are XOR-swizzled in 16-byte
-//     groups so that the fragment reads (ds_read_b128) hit distinct banks;
+//     two stages (three for the lower tiles); a slice row is one 128-byte cache line, so each
+//     load instruction touches 8 lines (the address unit's cost is per line touched); rows are
+//     XOR-swizzled in 16-byte groups so that the fragment reads (ds_read_b128) hit distinct
+//     banks;
 //   * one barrier per slice, between its two 32-wide steps; a step's 32 matrix instructions
 //     run token-block major and each carries a share of the rest: every token fragment is
 //     reloaded for the next step right after its last use (so only one token set is held),
@@ -33,10 +34,14 @@
 //     loop runs uniformly;
 //   * the output block goes through LDS and leaves as whole 16-byte row chunks, so each
 //     cache line of y is written by one store instruction;
+//   * tiles too few to fill the device split K: each workgroup writes its f32 sums in lane order
+//     and gemm_reduce_kernel adds them, split 0 first, and runs the epilogue;
+//   * at most kSkinnyTokens tokens go to gemm_skinny.hip;
 //   * workgroups are dealt to the 8 XCDs round robin; tiles are renumbered so that each XCD
 //     works through a compact group of tiles that share operand rows in its L2.
 // Generic kernel (any dtype, stride or alignment): LDS-tiled FMA loop with f32 accumulation
 // (f64 for f64 tensors).
+#include <algorithm>
 #include <type_traits>
 
 #include "cea_lds_dma.hpp"
@@ -46,23 +51,31 @@ namespace cea {
 namespace {
 
 constexpr int G_THREADS = 512;                       // 8 waves, two per SIMD
-constexpr int G_BM = 256;                            // tokens per tile
 constexpr int G_BW = 256;                            // weight rows per tile
 constexpr int G_BK = 64;                             // K per LDS slice
 constexpr int G_ROW = G_BK * 2;                      // bytes of one row of a slice: a cache line
-constexpr int G_NST = 2;                             // LDS stages
-constexpr int G_OPER = G_BM * G_ROW;                 // 32 KB per operand per slice
-constexpr int G_STAGE = 2 * G_OPER;                  // weight slice, then token slice
-constexpr int G_LDS = G_NST * G_STAGE;               // 128 KB
-constexpr int G_LOADS = G_OPER / (G_THREADS * 16);   // 16-byte loads per lane per operand
+constexpr int G_WBYTES = G_BW * G_ROW;               // weight part of a stage
+constexpr int G_WLOADS = G_WBYTES / (G_THREADS * 16);  // weight loads per wave and slice
 constexpr int kLgkm0 = 0xC07F;   // s_waitcnt lgkmcnt(0), vmcnt / expcnt left at their maximum
-static_assert(G_LOADS == 4 && G_BM == G_BW, "the load pattern assumes 4 x 8 rows per wave");
 
-// Tile (token block, weight block) of this workgroup.
-__device__ __forceinline__ void tile_of(const GemmParams& p, int& tm, int& tn) {
-  const int nwg = p.tiles_m * p.tiles_n;
+// TB: 16-token blocks per wave; a tile holds 2 waves of them.
+template <int TB> struct Tile {
+  static constexpr int BM = 32 * TB;                         // tokens per tile
+  static constexpr int STAGE = G_WBYTES + BM * G_ROW;        // weight slice, then token slice
+  static constexpr int NST = 160 * 1024 / STAGE >= 3 ? 3 : 2;  // LDS stages
+  static constexpr int LDS = NST * STAGE;
+  static constexpr int XLOADS = (TB + 1) / 2;   // token loads per wave (odd TB: the last by waves 0-3)
+  static constexpr int LOADS = G_WLOADS + XLOADS;
+};
+
+// Tile (token block, weight block) and K split of this workgroup.
+__device__ __forceinline__ void tile_of(const GemmParams& p, int& tm, int& tn, int& split) {
+  const int nwg = gridDim.x;
   int b = blockIdx.x;
   if ((nwg & 7) == 0) b = (b & 7) * (nwg >> 3) + (b >> 3);   // one contiguous run per XCD
+  const int tiles = p.tiles_m * p.tiles_n;
+  split = b / tiles;
+  b -= split * tiles;
   const int per_group = p.group_m * p.tiles_n;                // group_m token blocks wide
   const int grp = b / per_group;
   const int first = grp * p.group_m;
@@ -72,97 +85,101 @@ __device__ __forceinline__ void tile_of(const GemmParams& p, int& tm, int& tn) {
   tn = r / gm;
 }
 
-template <typename T, int MODE, int ACT>
+template <typename T, int MODE, int ACT, int TB>
 __global__ __launch_bounds__(G_THREADS, 1) void gemm_mfma_kernel(const GemmParams p) {
   typedef typename GMfma<T>::frag frag;
+  typedef Tile<TB> L;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   constexpr int ESZ = sizeof(T);
   constexpr int OUT_N = MODE == kGated ? G_BW / 2 : G_BW;   // output columns per tile
+  constexpr int NST = L::NST;
 
   const int tid = threadIdx.x;
-  const int wave = tid >> 6;
+  const int wave = uniform(tid >> 6);
   const int lane = tid & 63;
   const int wm = wave & 1;    // token half of the tile
   const int wn = wave >> 1;   // weight quarter (gated: output-column quarter)
-  int tm, tn;
-  tile_of(p, tm, tn);
-  const int m0 = tm * G_BM;
+  int tm, tn, split;
+  tile_of(p, tm, tn, split);
+  const int m0 = tm * L::BM;
   const int n0 = tn * OUT_N;
   const int K = p.K;
-  const int KT = (K + G_BK - 1) / G_BK;
+  const int s_begin = split * p.split_slices;
+  const int s_end = min((K + G_BK - 1) / G_BK, s_begin + p.split_slices);
+  const int kend = min(K, s_end * G_BK);
 
-  const int rows_x = min(G_BM, p.M - m0);
+  const int rows_x = min(L::BM, p.M - m0);
   const i32x4 rx = make_rsrc((const char*)p.x + (int64_t)m0 * p.ldx * ESZ,
                              (uint32_t)((int64_t)(rows_x - 1) * p.ldx * ESZ + (int64_t)K * ESZ));
-  i32x4 rw;
-  if constexpr (MODE == kGated) {   // waves 0-3 load the 128 gate rows, 4-7 the 128 up rows
-    const int rows = min(OUT_N, p.N - n0);
-    const char* base = (const char*)(wave < 4 ? p.wg : p.wu) + (int64_t)n0 * p.ldw * ESZ;
-    rw = make_rsrc(base, (uint32_t)((int64_t)(rows - 1) * p.ldw * ESZ + (int64_t)K * ESZ));
-  } else {
-    const int rows = min(G_BW, p.N - n0);
-    rw = make_rsrc((const char*)p.wg + (int64_t)n0 * p.ldw * ESZ,
-                   (uint32_t)((int64_t)(rows - 1) * p.ldw * ESZ + (int64_t)K * ESZ));
-  }
+  const int rows_w = min(OUT_N, p.N - n0);
+  const uint32_t wbytes = (uint32_t)((int64_t)(rows_w - 1) * p.ldw * ESZ + (int64_t)K * ESZ);
+  const i32x4 rg = make_rsrc((const char*)p.wg + (int64_t)n0 * p.ldw * ESZ, wbytes);
+  const i32x4 ru = MODE == kGated ? make_rsrc((const char*)p.wu + (int64_t)n0 * p.ldw * ESZ, wbytes) : rg;
 
-  // slice loads: wave w fills rows [32w, 32w + 32) of both operands, 8 rows x 128 bytes per
-  // instruction (same lane pattern and swizzle as the 4-wave kernel)
-  int kcol[2];
-  uint32_t off_w[G_LOADS], off_x[G_LOADS];
+  // slice loads: load i of wave w fills rows [64 i + 8 w, 64 i + 8 w + 8) of an operand, 8 rows x
+  // 128 bytes; the swizzle depends on the row modulo 16, so on the wave alone
+  const int lrow = 8 * wave + (lane >> 3);
+  const int grp = (lane & 7) ^ g_swz(lrow);
+  const int kcol = grp * 8;
+  uint32_t off_w[G_WLOADS], off_x[L::XLOADS];
 #pragma unroll
-  for (int i = 0; i < G_LOADS; ++i) {
-    const int row = 32 * wave + 8 * i + (lane >> 3);
-    const int grp = (lane & 7) ^ g_swz(row);
-    if (i < 2) kcol[i] = grp * 8;
-    const int wrow = MODE == kGated ? (row & 127) : row;
-    off_w[i] = (uint32_t)((int64_t)wrow * p.ldw * ESZ) + grp * 16;
-    off_x[i] = (uint32_t)((int64_t)row * p.ldx * ESZ) + grp * 16;
+  for (int i = 0; i < G_WLOADS; ++i) {   // gated: loads 0, 1 the 128 gate rows, 2, 3 the up rows
+    const int row = lrow + 64 * (MODE == kGated ? i & 1 : i);
+    off_w[i] = (uint32_t)((int64_t)row * p.ldw * ESZ) + grp * 16;
   }
-  const uint32_t lds_wave = lds_addr(smem) + wave * G_LOADS * 1024;
-  auto issue_one = [&](int s, int i) {   // i < G_LOADS: weight rows, else token rows
-    const uint32_t sb = lds_wave + (uint32_t)(s & (G_NST - 1)) * G_STAGE;
+#pragma unroll
+  for (int i = 0; i < L::XLOADS; ++i)
+    off_x[i] = (uint32_t)((int64_t)(lrow + 64 * i) * p.ldx * ESZ) + grp * 16;
+  const uint32_t lds_wave = lds_addr(smem) + wave * 1024;
+  auto issue_one = [&](int s, int stage, int i) {   // i < G_WLOADS: weight rows, else token rows
+    const uint32_t sb = lds_wave + (uint32_t)stage * L::STAGE;
     const uint32_t kb = (uint32_t)s * G_ROW;
-    const int li = i < G_LOADS ? i : i - G_LOADS;
-    const bool kin = s * G_BK + kcol[li & 1] < K;
-    if (i < G_LOADS)
-      buffer_load_lds16_m0_so(rw, sb + li * 1024, kin ? off_w[li] : kOutOfRange, kb);
-    else
-      buffer_load_lds16_m0_so(rx, sb + G_OPER + li * 1024, kin ? off_x[li] : kOutOfRange, kb);
+    const bool kin = s * G_BK + kcol < kend;
+    if (i < G_WLOADS) {
+      buffer_load_lds16_m0_so(MODE == kGated && i >= 2 ? ru : rg, sb + i * 8192,
+                              kin ? off_w[i] : kOutOfRange, kb);
+    } else {
+      const int li = i - G_WLOADS;
+      if ((TB & 1) && li == L::XLOADS - 1 && wave >= 4) return;
+      buffer_load_lds16_m0_so(rx, sb + G_WBYTES + li * 8192, kin ? off_x[li] : kOutOfRange, kb);
+    }
+  };
+  // this wave's loads of all but the newest slice have landed
+  auto wait_slice = [&] {
+    if constexpr (NST == 2) wait_vmcnt<0>();
+    else if (!(TB & 1) || wave < 4) wait_vmcnt<(NST - 2) * L::LOADS>();
+    else wait_vmcnt<(NST - 2) * (L::LOADS - 1)>();
   };
 
-  // fragments: 4 weight blocks (j < 4) and 8 token blocks (j >= 4) of 16 rows per step
+  // fragments: 4 weight blocks and TB token blocks of 16 rows per 32-wide step
   uint32_t rd[2];
 #pragma unroll
   for (int q = 0; q < 2; ++q)
     rd[q] = (lane & 15) * G_ROW + (((4 * q + (lane >> 4)) ^ g_swz(lane & 15)) << 4);
-  auto frag_row = [&](int j) {
-    if (j < 4)
-      return MODE == kGated ? (j >> 1) * 128 + wn * 32 + (j & 1) * 16 : wn * 64 + j * 16;
-    return G_BM + wm * 128 + (j - 4) * 16;
+  auto read_a = [&](int stage, int q, int j, frag (&fa)[4]) {
+    const int row = MODE == kGated ? (j >> 1) * 128 + wn * 32 + (j & 1) * 16 : wn * 64 + j * 16;
+    fa[j] = *(const frag*)(smem + stage * L::STAGE + rd[q] + row * G_ROW);
   };
-  auto read_a = [&](int s, int q, int j, frag (&fa)[4]) {
-    fa[j] = *(const frag*)(smem + (s & (G_NST - 1)) * G_STAGE + rd[q] + frag_row(j) * G_ROW);
-  };
-  auto read_b = [&](int s, int q, int t, frag (&fb)[8]) {
-    fb[t] = *(const frag*)(smem + (s & (G_NST - 1)) * G_STAGE + rd[q] + frag_row(4 + t) * G_ROW);
+  auto read_b = [&](int stage, int q, int t, frag (&fb)[TB]) {
+    fb[t] = *(const frag*)(smem + stage * L::STAGE + G_WBYTES + rd[q] + (wm * (16 * TB) + t * 16) * G_ROW);
   };
 
-  f32x4 acc[4][8];
+  f32x4 acc[4][TB];
 #pragma unroll
   for (int f = 0; f < 4; ++f)
 #pragma unroll
-    for (int t = 0; t < 8; ++t)
+    for (int t = 0; t < TB; ++t)
 #pragma unroll
       for (int e = 0; e < 4; ++e) acc[f][t][e] = 0.0f;
 
-  // One 32-wide step: 32 matrix instructions token-block major; each token fragment is
-  // reloaded for the next step (slice rs, step rq) right after its last use, the next
-  // weight fragments go into the other set early, and with DMA the 8 refill loads of slice
-  // s + 2 are spread one per 4 instructions.
-  frag fa0[4], fa1[4], fb[8];
-  auto step = [&](int s, const frag (&fa)[4], int rs, int rq, frag (&na)[4], auto dma) {
+  // One 32-wide step: 4 TB matrix instructions token-block major; each token fragment is
+  // reloaded for the next step (stage rs, step rq) right after its last use, the next
+  // weight fragments go into the other set early, and with DMA the loads of slice ls (into
+  // stage lst) are spread evenly.
+  frag fa0[4], fa1[4], fb[TB];
+  auto step = [&](const frag (&fa)[4], int rs, int rq, frag (&na)[4], auto dma, int ls, int lst) {
 #pragma unroll
-    for (int t = 0; t < 8; ++t)
+    for (int t = 0; t < TB; ++t)
 #pragma unroll
       for (int f = 0; f < 4; ++f) {
         const int i = t * 4 + f;
@@ -170,32 +187,50 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm_mfma_kernel(const GemmParam
         if (f == 3) read_b(rs, rq, t, fb);
         if ((i & 3) == 1 && i < 16) read_a(rs, rq, i >> 2, na);
         if constexpr (decltype(dma)::value) {
-          if ((i & 3) == 2) issue_one(s + G_NST, i >> 2);
+#pragma unroll
+          for (int l = 0; l < L::LOADS; ++l)
+            if (i == l * 4 * TB / L::LOADS + 2) issue_one(ls, lst, l);
         }
         __builtin_amdgcn_sched_barrier(0);
       }
   };
 
 #pragma unroll
-  for (int s = 0; s < G_NST; ++s)
+  for (int s = 0; s < NST; ++s)
 #pragma unroll
-    for (int i = 0; i < 2 * G_LOADS; ++i) issue_one(s, i);
-  wait_vmcnt<2 * G_LOADS>();
+    for (int i = 0; i < L::LOADS; ++i) issue_one(s_begin + s, s, i);
+  if (!(TB & 1) || wave < 4) wait_vmcnt<(NST - 1) * L::LOADS>();
+  else wait_vmcnt<(NST - 1) * (L::LOADS - 1)>();
   barrier_no_fence();
 #pragma unroll
   for (int j = 0; j < 4; ++j) read_a(0, 0, j, fa0);
 #pragma unroll
-  for (int t = 0; t < 8; ++t) read_b(0, 0, t, fb);
+  for (int t = 0; t < TB; ++t) read_b(0, 0, t, fb);
   __builtin_amdgcn_sched_barrier(0);
-  for (int s = 0; s < KT; ++s) {
-    step(s, fa0, s, 1, fa1, std::integral_constant<bool, false>());
-    wait_vmcnt<0>();
+  int st = 0;   // stage of slice s
+  for (int s = s_begin; s < s_end; ++s) {
+    step(fa0, st, 1, fa1, std::integral_constant<bool, false>(), 0, 0);
+    wait_slice();
     __builtin_amdgcn_s_waitcnt(kLgkm0);
     barrier_no_fence();
     __builtin_amdgcn_sched_barrier(0);
-    step(s, fa1, s + 1, 0, fa0, std::integral_constant<bool, true>());
+    const int nx = NST == 2 ? st ^ 1 : (st == NST - 1 ? 0 : st + 1);
+    step(fa1, nx, 0, fa0, std::integral_constant<bool, true>(), s + NST, st);
+    st = nx;
   }
   wait_vmcnt<0>();
+
+  if (p.partial != nullptr) {
+    // one of several K splits: the raw sums, 1 KB per 16 x 16 block in lane order, for
+    // gemm_reduce_kernel
+    f32x4* dst = (f32x4*)p.partial +
+                 ((((int64_t)split * p.tiles_n + tn) * p.tiles_m + tm) * 8 + wave) * (4 * TB * 64) + lane;
+#pragma unroll
+    for (int f = 0; f < 4; ++f)
+#pragma unroll
+      for (int t = 0; t < TB; ++t) dst[(f * TB + t) * 64] = acc[f][t];
+    return;
+  }
 
   // epilogue: block (f, t) holds token t * 16 + (l & 15) and weight rows f * 16 + 4 (l >> 4) ..
   const int q4 = lane >> 4;
@@ -221,7 +256,7 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm_mfma_kernel(const GemmParam
     auto row_swz = [](int r) { return CPR == 8 ? ((r >> 1) & 7) : ((r >> 2) & 3); };
     __builtin_amdgcn_s_waitcnt(kLgkm0);
     barrier_no_fence();
-    char* stage = smem + wave * (128 * RB);
+    char* stage = smem + wave * (16 * TB * RB);
     auto to_lds = [&](auto bias) {
 #pragma unroll
       for (int f = 0; f < NF; ++f) {
@@ -232,7 +267,7 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm_mfma_kernel(const GemmParam
           if constexpr (MODE == kGated) bias4<T, float>(p.bu, col0 + c4, p.N, true, buv);
         }
 #pragma unroll
-        for (int t = 0; t < 8; ++t) {
+        for (int t = 0; t < TB; ++t) {
           float v[4];
           values(f, t, bgv, buv, v, bias);
           T o[4];
@@ -249,11 +284,11 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm_mfma_kernel(const GemmParam
     if (p.bg != nullptr) to_lds(std::integral_constant<bool, true>());
     else to_lds(std::integral_constant<bool, false>());
 #pragma unroll
-    for (int k = 0; k < 128 / RPI; ++k) {
+    for (int k = 0; k < 16 * TB / RPI; ++k) {
       const int row = k * RPI + lane / CPR;
       const int c = lane % CPR;
       const uint4 raw = *(const uint4*)(stage + row * RB + ((c ^ row_swz(row)) * 16));
-      const int tok = m0 + wm * 128 + row;
+      const int tok = m0 + wm * (16 * TB) + row;
       const int col = col0 + c * 8;
       if (tok < p.M && col < p.N) *(uint4*)(y + (int64_t)tok * p.ldy + col) = raw;
     }
@@ -267,14 +302,53 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm_mfma_kernel(const GemmParam
     bias4<T, float>(p.bg, col, p.N, vec, bgv);
     if constexpr (MODE == kGated) bias4<T, float>(p.bu, col, p.N, vec, buv);
 #pragma unroll
-    for (int t = 0; t < 8; ++t) {
-      const int tok = m0 + wm * 128 + t * 16 + (lane & 15);
+    for (int t = 0; t < TB; ++t) {
+      const int tok = m0 + wm * (16 * TB) + t * 16 + (lane & 15);
       if (tok >= p.M) continue;
       float v[4];
       values(f, t, bgv, buv, v, std::integral_constant<bool, true>());
       store4<T, float>(y + (int64_t)tok * p.ldy, col, p.N, vec, v);
     }
   }
+}
+
+// The sum of a split launch's partials (split 0 first) and the epilogue: one wave per 16 x 16
+// block, in the layout the tiles wrote, so the reads (all but a few percent of the bytes) are
+// whole kilobytes.  Bound by those reads, which mostly still sit in the Infinity Cache: 42 MB of
+// partials (300 tokens x 4096 x 14336, 8 splits) add about 10 us to a call of 50 us that took
+// 285 us unsplit.
+template <typename T, int MODE, int ACT>
+__global__ __launch_bounds__(256) void gemm_reduce_kernel(const GemmParams p, int tb, int splits) {
+  const int lane = threadIdx.x & 63;
+  const int nf = MODE == kGated ? 2 : 4;   // output column blocks of a tile's wave
+  const int per_wave = nf * tb;
+  const int64_t blk = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int64_t tw = blk / per_wave;       // (weight block, token block, wave) of the tile grid
+  const int r = (int)(blk - tw * per_wave);
+  const int f = r / tb, t = r - f * tb;
+  const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n;
+  if (tw >= tiles * 8) return;
+  const int wave = (int)(tw & 7);
+  const int tm = (int)((tw >> 3) % p.tiles_m), tn = (int)((tw >> 3) / p.tiles_m);
+  const int tok = tm * 32 * tb + (wave & 1) * 16 * tb + t * 16 + (lane & 15);
+  const int col = tn * (nf * 64) + (wave >> 1) * (nf * 16) + f * 16 + 4 * (lane >> 4);
+  if (tok >= p.M || col >= p.N) return;
+  const int64_t per_split = tiles * 8 * (4 * tb * 64);
+  const f32x4* src = (const f32x4*)p.partial + tw * (4 * tb * 64) + (f * tb + t) * 64 + lane;
+  f32x4 g = src[0], u = {0.0f, 0.0f, 0.0f, 0.0f};
+  if constexpr (MODE == kGated) u = src[2 * tb * 64];
+  for (int i = 1; i < splits; ++i) {
+    g += src[i * per_split];
+    if constexpr (MODE == kGated) u += src[i * per_split + 2 * tb * 64];
+  }
+  const bool vec = p.vec_out != 0;
+  float gv[4], uv[4], bgv[4], buv[4] = {0.0f, 0.0f, 0.0f, 0.0f}, v[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) gv[j] = g[j], uv[j] = u[j];
+  bias4<T, float>(p.bg, col, p.N, vec, bgv);
+  if constexpr (MODE == kGated) bias4<T, float>(p.bu, col, p.N, vec, buv);
+  finish4<T, MODE, ACT, true, float>(gv, uv, bgv, buv, v);
+  store4<T, float>((T*)p.y + (int64_t)tok * p.ldy, col, p.N, vec, v);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -367,7 +441,47 @@ __global__ __launch_bounds__(256) void gemm_generic_kernel(const GemmParams p) {
 // ---------------------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------------------
-int g_group_m = 8;   // token blocks per tile group
+constexpr int kGroupM = 8;   // token blocks per tile group
+
+// Tile height and K splits of a launch.
+struct TilePlan {
+  int tb, splits, split_slices;
+  size_t ws;   // bytes of partial sums
+};
+constexpr size_t kMaxPartials = (size_t)128 << 20;
+
+// The launch of least modelled time: rounds of workgroups over the compute units, times the
+// slices each walks at its tile height's pace, plus the partial sums' way out and back.  Measured
+// pace (us per 64-wide slice with every unit busy): 0.94 / 1.11 / 1.69 at 128 / 160 / 256 tokens;
+// 192 (1.41) and 224 (1.50) are slower per token than 256 and are not built.  A small tile wins
+// where 256 tokens leave a last round nearly empty or pad much (3001 x 6144 x 4096: 288 tiles in
+// two rounds 172 us, 456 of 160 tokens 136 us; 300 tokens x 2 x 14336: 105 -> 81 us), splits
+// where the tiles are fewer than the units (4096 x 14336, 300 tokens: 32 tiles unsplit 163 us
+// and up, 8 splits 51 us).  A split keeps at least 512 of K.
+TilePlan plan_tiles(int64_t M, int64_t rows, int64_t K, size_t ws_bytes) {
+  static constexpr struct { int tb; double pace; } kHeights[] = {{8, 1.69}, {5, 1.11}, {4, 0.94}};
+  constexpr double kEnds = 5.0;      // prologue and epilogue of a workgroup, us
+  constexpr double kLaunch = 3.0;    // the reduction's launch, us
+  constexpr double kBytesUs = 6e6;   // partial sums written or read, bytes per us
+  const int cus = device_cus() > 0 ? device_cus() : 256;
+  const int kt = (int)((K + G_BK - 1) / G_BK);
+  TilePlan best{8, 1, kt, 0};
+  double least = 0;
+  for (const auto& h : kHeights) {
+    const int64_t tiles = ((M + 32 * h.tb - 1) / (32 * h.tb)) * ((rows + G_BW - 1) / G_BW);
+    for (int want = 1; want <= 16; ++want) {
+      const int slices = (kt + want - 1) / want;
+      if (want > 1 && (slices < 8 || tiles * want > 2 * cus)) break;
+      const int splits = want == 1 ? 1 : (kt + slices - 1) / slices;
+      const size_t ws = splits == 1 ? 0 : (size_t)(tiles * splits) * (size_t)(32 * h.tb * G_BW * 4);
+      if (ws > std::min(ws_bytes, kMaxPartials)) break;
+      const double rounds = (double)((tiles * splits + cus - 1) / cus);
+      const double us = rounds * (slices * h.pace + kEnds) + (splits > 1 ? kLaunch + 2.0 * ws / kBytesUs : 0);
+      if (least == 0 || us < least) least = us, best = {h.tb, splits, slices, ws};
+    }
+  }
+  return best;
+}
 
 bool mfma_path(const GemmParams& p, int dtype, int mode) {
   if (dtype != CEA_BF16 && dtype != CEA_F16) return false;
@@ -377,28 +491,49 @@ bool mfma_path(const GemmParams& p, int dtype, int mode) {
   // every byte offset of a tile's rows must stay below the out-of-range marker
   const int64_t lim = (int64_t)kOutOfRange;
   const int wrows = mode == kGated ? G_BW / 2 : G_BW;
-  if ((int64_t)(G_BM - 1) * p.ldx * 2 + (int64_t)p.K * 2 >= lim) return false;
+  if ((int64_t)(Tile<8>::BM - 1) * p.ldx * 2 + (int64_t)p.K * 2 >= lim) return false;
   if ((int64_t)(wrows - 1) * p.ldw * 2 + (int64_t)p.K * 2 >= lim) return false;
   return true;
+}
+
+template <typename T, int MODE, int ACT, int TB>
+int launch_tiles(GemmParams p, const TilePlan& pl, hipStream_t st) {
+  typedef Tile<TB> L;
+  const int out_n = MODE == kGated ? G_BW / 2 : G_BW;
+  p.tiles_m = (p.M + L::BM - 1) / L::BM;
+  p.tiles_n = (p.N + out_n - 1) / out_n;
+  p.group_m = kGroupM;
+  p.split_slices = pl.split_slices;
+  const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n;
+  CEA_REQUIRE(tiles * pl.splits <= INT32_MAX, CEA_EUNSUPPORTED, "linear: problem too large");
+  if (pl.splits == 1) p.partial = nullptr;
+  const hipError_t e = reserve_lds<gemm_mfma_kernel<T, MODE, ACT, TB>>(L::LDS);
+  CEA_REQUIRE(e == hipSuccess, CEA_ELAUNCH, "linear: cannot reserve %d bytes of LDS: %s", L::LDS,
+              hipGetErrorString(e));
+  hipLaunchKernelGGL((gemm_mfma_kernel<T, MODE, ACT, TB>), dim3((unsigned)(tiles * pl.splits)),
+                     dim3(G_THREADS), L::LDS, st, p);
+  CEA_CHECK_LAUNCH(MODE == kGated ? "linear_gated" : "linear");
+  if (pl.splits > 1) {
+    const int64_t blocks = tiles * 8 * (MODE == kGated ? 2 : 4) * TB;
+    hipLaunchKernelGGL((gemm_reduce_kernel<T, MODE, ACT>), dim3((unsigned)((blocks + 3) / 4)),
+                       dim3(256), 0, st, p, TB, pl.splits);
+    CEA_CHECK_LAUNCH(MODE == kGated ? "linear_gated" : "linear");
+  }
+  return CEA_OK;
 }
 
 template <typename T, int MODE, int ACT>
 int launch_one(GemmParams p, bool mfma, hipStream_t st) {
   if constexpr (sizeof(T) == 2) {
     if (mfma) {
-      const int out_n = MODE == kGated ? G_BW / 2 : G_BW;
-      p.tiles_m = (p.M + G_BM - 1) / G_BM;
-      p.tiles_n = (p.N + out_n - 1) / out_n;
-      p.group_m = g_group_m;
-      const int64_t total = (int64_t)p.tiles_m * p.tiles_n;
-      CEA_REQUIRE(total <= INT32_MAX, CEA_EUNSUPPORTED, "linear: problem too large");
-      const hipError_t e = reserve_lds<gemm_mfma_kernel<T, MODE, ACT>>(G_LDS);
-      CEA_REQUIRE(e == hipSuccess, CEA_ELAUNCH, "linear: cannot reserve %d bytes of LDS: %s",
-                  G_LDS, hipGetErrorString(e));
-      hipLaunchKernelGGL((gemm_mfma_kernel<T, MODE, ACT>), dim3((unsigned)total),
-                         dim3(G_THREADS), G_LDS, st, p);
-      CEA_CHECK_LAUNCH(MODE == kGated ? "linear_gated" : "linear");
-      return CEA_OK;
+      const int64_t rows = (int64_t)p.N * (MODE == kGated ? 2 : 1);
+      const bool ws16 = ((uintptr_t)p.partial & 15) == 0;
+      const TilePlan pl = plan_tiles(p.M, rows, p.K, p.partial && ws16 ? p.ws_bytes : 0);
+      switch (pl.tb) {
+        case 4: return launch_tiles<T, MODE, ACT, 4>(p, pl, st);
+        case 5: return launch_tiles<T, MODE, ACT, 5>(p, pl, st);
+        default: return launch_tiles<T, MODE, ACT, 8>(p, pl, st);
+      }
     }
   }
   const int64_t gy = (p.M + GG_T - 1) / GG_T;
@@ -429,8 +564,10 @@ int launch_typed(const GemmParams& p, int mode, int act, bool mfma, hipStream_t 
 // dtypes validated by the caller.  mode: 0 plain (w_up / b_up unused), 1 gated.
 int launch_linear(const cea_tensor* x, const cea_tensor* wg, const cea_tensor* wu,
                   const cea_tensor* bg, const cea_tensor* bu, cea_tensor* y, int mode, int act,
-                  hipStream_t st) {
+                  void* ws, size_t ws_bytes, hipStream_t st) {
   GemmParams p{};
+  p.partial = (float*)ws;
+  p.ws_bytes = ws ? ws_bytes : 0;
   p.x = x->data;
   p.wg = wg->data;
   p.wu = wu ? wu->data : nullptr;
@@ -461,6 +598,11 @@ int launch_linear(const cea_tensor* x, const cea_tensor* wg, const cea_tensor* w
   }
   set_error("linear: unsupported dtype %s", dtype_name(x->dtype));
   return CEA_EUNSUPPORTED;
+}
+
+size_t linear_workspace_bytes(int64_t M, int64_t N, int64_t K, int dtype, int mode) {
+  if ((dtype != CEA_BF16 && dtype != CEA_F16) || M <= kSkinnyTokens || K % 8) return 0;
+  return plan_tiles(M, N * (mode == kGated ? 2 : 1), K, SIZE_MAX).ws;
 }
 
 }  // namespace cea

@@ -17,6 +17,11 @@ struct GemmParams {
   int32_t M, N, K;  // N = output columns
   int32_t tiles_m, tiles_n, group_m;
   int32_t vec_out;  // 2: 16-byte row chunks, 1: 4-element stores, 0: element stores
+  // K splits of the tile kernel: 64-wide slices per split, f32 sums (null: one split) and the
+  // caller's scratch size
+  int32_t split_slices;
+  float* partial;
+  size_t ws_bytes;
 };
 
 // Rows of x the skinny kernel takes (4 blocks of 16).

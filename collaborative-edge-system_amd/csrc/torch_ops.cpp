@@ -456,18 +456,24 @@ std::vector<int64_t> out_shape(const Tensor& x, int64_t n) {
   return s;
 }
 
+// The scratch of a projection to n columns (undefined when it needs none).
+Tensor linear_workspace(const Tensor& x2, int64_t n, int gated, const at::Device& dev) {
+  const size_t bytes =
+      cea_linear_workspace_bytes(x2.size(0), n, x2.size(1), code_of(x2.scalar_type()), gated);
+  return bytes ? workspace(bytes, dev) : Tensor();
+}
+
 void linear_call(const Tensor& x2, const Tensor& weight, const c10::optional<Tensor>& bias,
                  const Tensor& y2, const at::Device& dev) {
   const Tensor w = inner(weight);
   const Tensor b = bias ? inner(*bias) : Tensor();
   c10::DeviceGuard guard(dev);
-  cea_tensor a = arg(x2), c = arg(w), e = arg(y2);
-  if (b.defined()) {
-    cea_tensor d = arg(b);
-    check_rc(cea_linear(&a, &c, &d, &e, stream_of(dev)), "linear");
-  } else {
-    check_rc(cea_linear(&a, &c, nullptr, &e, stream_of(dev)), "linear");
-  }
+  const Tensor ws = linear_workspace(x2, w.size(0), 0, dev);
+  cea_tensor a = arg(x2), c = arg(w), d, e = arg(y2);
+  if (b.defined()) d = arg(b);
+  check_rc(cea_linear_ws(&a, &c, b.defined() ? &d : nullptr, &e, ws.defined() ? ws.data_ptr() : nullptr,
+                         ws.defined() ? (size_t)ws.numel() : 0, stream_of(dev)),
+           "linear");
 }
 
 Tensor linear(const Tensor& x, const Tensor& weight, const c10::optional<Tensor>& bias) {
@@ -507,8 +513,10 @@ Tensor linear_gated(const Tensor& x, const Tensor& w_gate, const Tensor& w_up,
   cea_tensor f, g;
   if (bg.defined()) f = arg(bg);
   if (bu.defined()) g = arg(bu);
-  check_rc(cea_linear_gated(&a, &c, &d, bg.defined() ? &f : nullptr, bu.defined() ? &g : nullptr, &e,
-                            (int32_t)act, stream_of(dev)),
+  const Tensor ws = linear_workspace(x2, w_gate.size(0), 1, dev);
+  check_rc(cea_linear_gated_ws(&a, &c, &d, bg.defined() ? &f : nullptr, bu.defined() ? &g : nullptr, &e,
+                               (int32_t)act, ws.defined() ? ws.data_ptr() : nullptr,
+                               ws.defined() ? (size_t)ws.numel() : 0, stream_of(dev)),
            "linear_gated");
   return y;
 }

@@ -297,3 +297,33 @@ def test_linear_few_tokens(cea, dev, dtype, m, k, n):
     chain = cea.layers.gated_mul(out[:, 8:8 + n].contiguous(), out[:, 8 + n:8 + 2 * n].contiguous(), "silu")
     torch.cuda.synchronize()
     _same_as_chain(y, chain, f"few tokens gated {m}x{k}x{n} {dtype}")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,k,n", [
+    (97, 1032, 68),     # 128-token tiles, two K splits, the second with a K tail of 8
+    (161, 1096, 4100),  # one token past a 160-token tile; N not a multiple of 8
+    (300, 2056, 132),   # more splits than slices divide into evenly
+    (129, 512, 64),     # K too short to split
+])
+def test_linear_tile_heights_and_splits(cea, dev, dtype, m, k, n):
+    """Tile heights below 256 tokens and K splits, plain and gated, through the operator (with
+    scratch) and through the C entry point without scratch (unsplit)."""
+    g = torch.Generator().manual_seed(m + 3 * k + n)
+    x, w, b = _operands(g, m, k, 2 * n, dtype)
+    xd, wd, bd = x.to(dev), w.to(dev), b.to(dev)
+    y = cea.projection.linear(xd, wd, bd)
+    torch.cuda.synchronize()
+    _check_linear(y, x, w, b, f"tiles {m}x{k}x{n} {dtype}")
+    act = cea.projection.linear_gated(xd, wd[:n], wd[n:], bd[:n], bd[n:], "silu")
+    chain = cea.layers.gated_mul(y[:, :n], y[:, n:], "silu")
+    torch.cuda.synchronize()
+    _same_as_chain(act, chain, f"tiles gated {m}x{k}x{n} {dtype}")
+    import ctypes
+    nat = cea._native
+    u = torch.empty_like(y)
+    rc = nat.load_library().cea_linear(*(ctypes.byref(nat.tensor_arg(t)) for t in (xd, wd, bd, u)),
+                                       nat.stream_of(xd.device))
+    torch.cuda.synchronize()
+    assert rc == 0, nat.last_error()
+    _check_linear(u, x, w, b, f"tiles without scratch {m}x{k}x{n} {dtype}")
