@@ -36,7 +36,7 @@
 //     cache line of y is written by one store instruction;
 //   * tiles too few to fill the device split K: each workgroup writes its f32 sums in lane order
 //     and gemm_reduce_kernel adds them, split 0 first, and runs the epilogue;
-//   * at most kSkinnyTokens tokens go to gemm_skinny.hip;
+//   * at most kSkinnyTokens tokens, and f32 operands, go to gemm_skinny.hip;
 //   * workgroups are dealt to the 8 XCDs round robin; tiles are renumbered so that each XCD
 //     works through a compact group of tiles that share operand rows in its L2.
 // Generic kernel (any dtype, stride or alignment): LDS-tiled FMA loop with f32 accumulation
@@ -484,15 +484,16 @@ TilePlan plan_tiles(int64_t M, int64_t rows, int64_t K, size_t ws_bytes) {
 }
 
 bool mfma_path(const GemmParams& p, int dtype, int mode) {
-  if (dtype != CEA_BF16 && dtype != CEA_F16) return false;
-  if (p.K % 8 || p.ldx % 8 || p.ldw % 8) return false;
+  if (dtype != CEA_BF16 && dtype != CEA_F16 && dtype != CEA_F32) return false;
+  const int64_t esz = dtype_size(dtype), per16 = 16 / esz;
+  if (p.K % per16 || p.ldx % per16 || p.ldw % per16) return false;
   auto al16 = [](const void* q) { return ((uintptr_t)q & 15) == 0; };
   if (!al16(p.x) || !al16(p.wg) || (mode == kGated && !al16(p.wu))) return false;
   // every byte offset of a tile's rows must stay below the out-of-range marker
   const int64_t lim = (int64_t)kOutOfRange;
   const int wrows = mode == kGated ? G_BW / 2 : G_BW;
-  if ((int64_t)(Tile<8>::BM - 1) * p.ldx * 2 + (int64_t)p.K * 2 >= lim) return false;
-  if ((int64_t)(wrows - 1) * p.ldw * 2 + (int64_t)p.K * 2 >= lim) return false;
+  if ((int64_t)(Tile<8>::BM - 1) * p.ldx * esz + (int64_t)p.K * esz >= lim) return false;
+  if ((int64_t)(wrows - 1) * p.ldw * esz + (int64_t)p.K * esz >= lim) return false;
   return true;
 }
 
@@ -589,7 +590,8 @@ int launch_linear(const cea_tensor* x, const cea_tensor* wg, const cea_tensor* w
   p.vec_out = v16 ? 2 : v8 ? 1 : 0;
   if (p.M == 0 || p.N == 0) return CEA_OK;
   const bool mfma = mfma_path(p, x->dtype, mode);
-  if (mfma && p.M <= kSkinnyTokens) return launch_linear_skinny(p, x->dtype, mode, act, st);
+  if (mfma && (p.M <= kSkinnyTokens || x->dtype == CEA_F32))
+    return launch_linear_skinny(p, x->dtype, mode, act, st);
   switch (x->dtype) {
     case CEA_BF16: return launch_typed<bf16>(p, mode, act, mfma, st);
     case CEA_F16: return launch_typed<f16>(p, mode, act, mfma, st);

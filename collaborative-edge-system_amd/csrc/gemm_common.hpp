@@ -26,7 +26,7 @@ struct GemmParams {
 
 // Rows of x the skinny kernel takes (4 blocks of 16).
 constexpr int kSkinnyTokens = 64;
-// Operands as gemm.hip's matrix-core path, M <= kSkinnyTokens, bf16 / f16.
+// Operands as gemm.hip's matrix-core path; bf16 / f16 with M <= kSkinnyTokens, or f32.
 int launch_linear_skinny(const GemmParams& p, int dtype, int mode, int act, hipStream_t st);
 
 namespace {
@@ -50,6 +50,15 @@ template <> struct GMfma<f16> {
 };
 
 enum { kPlain = 0, kGated = 1 };
+// f32: a fragment holds 4 consecutive K per lane, multiplied in 4 steps of v_mfma_f32_16x16x4.
+template <> struct GMfma<float> {
+  typedef f32x4 frag;
+  static __device__ __forceinline__ f32x4 run(frag a, frag b, f32x4 c) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], b[j], c, 0, 0, 0);
+    return c;
+  }
+};
 
 constexpr uint32_t kOutOfRange = 0x80000000u;        // above every resource's range
 

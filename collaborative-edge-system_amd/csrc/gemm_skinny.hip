@@ -1,5 +1,6 @@
 // Projections of few tokens (decode steps) on gfx950 matrix cores: y = x . w^T and the gated
-// gate/up form of gemm.hip, for at most kSkinnyTokens rows of x.
+// gate/up form of gemm.hip, for at most kSkinnyTokens rows of x; and f32 projections of any
+// number of tokens, with true f32 products (v_mfma_f32_16x16x4).
 //
 // Bound by reading the weight once.  gemm.hip's 256 x 256 tiles leave most of the device idle
 // here (4096 x 14336: 16 workgroups, each walking all of K: 293 us at 32 tokens); this kernel
@@ -25,8 +26,7 @@ namespace {
 
 constexpr int S_WAVES = 8;
 constexpr int S_THREADS = S_WAVES * 64;
-constexpr int S_BK = 64;   // K per slice
-constexpr int S_ROW = S_BK * 2;   // bytes of a slice row: a cache line
+constexpr int S_ROW = 128;   // bytes of a slice row: a cache line (64 of K in 16 bits, 32 in f32)
 
 // RB: 16-row weight blocks of a workgroup (gated: RB / 2 of the gate and the matching RB / 2 of
 // the up rows), TB: 16-token blocks of x.
@@ -43,6 +43,7 @@ __global__ __launch_bounds__(S_THREADS, 2) void gemm_skinny_kernel(const GemmPar
   typedef typename GMfma<T>::frag frag;
   typedef SkinnyLds<RB, TB> L;
   constexpr int ESZ = sizeof(T);
+  constexpr int BK = S_ROW / ESZ;   // K per slice
   constexpr int NB = MODE == kGated ? RB / 2 : RB;   // output column blocks
   constexpr int PD = L::PD;
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -51,10 +52,13 @@ __global__ __launch_bounds__(S_THREADS, 2) void gemm_skinny_kernel(const GemmPar
   const int lane = threadIdx.x & 63;
   const int n0 = blockIdx.x * NB * 16;
   const int K = p.K;
-  const int KT = (K + S_BK - 1) / S_BK;
+  const int KT = (K + BK - 1) / BK;
   const int rows = min(NB * 16, p.N - n0);
+  const int m0 = blockIdx.y * TB * 16;
+  const int toks = min(TB * 16, p.M - m0);
 
-  const i32x4 rx = make_rsrc(p.x, (uint32_t)((int64_t)(p.M - 1) * p.ldx * ESZ + (int64_t)K * ESZ));
+  const i32x4 rx = make_rsrc((const char*)p.x + (int64_t)m0 * p.ldx * ESZ,
+                             (uint32_t)((int64_t)(toks - 1) * p.ldx * ESZ + (int64_t)K * ESZ));
   const uint32_t wbytes = (uint32_t)((int64_t)(rows - 1) * p.ldw * ESZ + (int64_t)K * ESZ);
   const i32x4 rg = make_rsrc((const char*)p.wg + (int64_t)n0 * p.ldw * ESZ, wbytes);
   const i32x4 ru = MODE == kGated ? make_rsrc((const char*)p.wu + (int64_t)n0 * p.ldw * ESZ, wbytes) : rg;
@@ -66,7 +70,7 @@ __global__ __launch_bounds__(S_THREADS, 2) void gemm_skinny_kernel(const GemmPar
   for (int i = 0; i < 2; ++i) {
     const int row = 8 * i + (lane >> 3);
     const int grp = (lane & 7) ^ g_swz(row);
-    kcol[i] = grp * 8;
+    kcol[i] = grp * (16 / ESZ);
     off_w[i] = (uint32_t)((int64_t)row * p.ldw * ESZ) + grp * 16;
     off_x[i] = (uint32_t)((int64_t)row * p.ldx * ESZ) + grp * 16;
   }
@@ -76,7 +80,7 @@ __global__ __launch_bounds__(S_THREADS, 2) void gemm_skinny_kernel(const GemmPar
   auto load = [&](int d, int s) {   // slice s into ring stage d
     const uint32_t kb = (uint32_t)s * S_ROW;
     const uint32_t base = ring_lds + (uint32_t)d * L::SLICE;
-    const bool kin[2] = {s * S_BK + kcol[0] < K, s * S_BK + kcol[1] < K};
+    const bool kin[2] = {s * BK + kcol[0] < K, s * BK + kcol[1] < K};
 #pragma unroll
     for (int f = 0; f < RB; ++f)
 #pragma unroll
@@ -150,7 +154,7 @@ __global__ __launch_bounds__(S_THREADS, 2) void gemm_skinny_kernel(const GemmPar
 #pragma unroll
       for (int w = 1; w < S_WAVES; ++w) u += red[w][NB * TB + i][lane];
     }
-    const int tok = t * 16 + (lane & 15);
+    const int tok = m0 + t * 16 + (lane & 15);
     const int col = n0 + f * 16 + 4 * (lane >> 4);
     if (tok >= p.M || col >= p.N) continue;
     float gv[4], uv[4], bgv[4], buv[4] = {0.0f, 0.0f, 0.0f, 0.0f}, v[4];
@@ -170,7 +174,7 @@ int launch_shape(const GemmParams& p, hipStream_t st) {
   const hipError_t e = reserve_lds<gemm_skinny_kernel<T, MODE, ACT, RB, TB>>(lds);
   CEA_REQUIRE(e == hipSuccess, CEA_ELAUNCH, "linear: cannot reserve %d bytes of LDS: %s", lds,
               hipGetErrorString(e));
-  hipLaunchKernelGGL((gemm_skinny_kernel<T, MODE, ACT, RB, TB>), dim3(ceil_div(p.N, NB * 16)),
+  hipLaunchKernelGGL((gemm_skinny_kernel<T, MODE, ACT, RB, TB>), dim3(ceil_div(p.N, NB * 16), ceil_div(p.M, TB * 16)),
                      dim3(S_THREADS), lds, st, p);
   CEA_CHECK_LAUNCH(MODE == kGated ? "linear_gated" : "linear");
   return CEA_OK;
@@ -194,8 +198,8 @@ template <int MODE> int weight_blocks(const GemmParams& p) {
 }
 
 template <typename T, int MODE, int ACT, int RB>
-int launch_blocks(const GemmParams& p, hipStream_t st) {
-  switch (ceil_div(p.M, 16)) {
+int launch_tokens(const GemmParams& p, int tb, hipStream_t st) {
+  switch (tb) {
     case 1: return launch_shape<T, MODE, ACT, RB, 1>(p, st);
     case 2: return launch_shape<T, MODE, ACT, RB, 2>(p, st);
     case 3: return launch_shape<T, MODE, ACT, RB, 3>(p, st);
@@ -203,13 +207,45 @@ int launch_blocks(const GemmParams& p, hipStream_t st) {
   }
 }
 
+// f32: weight and token blocks per workgroup.  A compute unit needs about 36 ns per block pair
+// and slice for the matrix instructions and 36 ns per block for its 2 KB; a round of workgroups
+// costs about 2 us more for its first loads and its sums.  Measured (us, generic kernel before ->
+// this rule; RB x TB 2 x 2 / 2 x 3 / 4 x 4): 512 tokens 1536 x 512 73 -> 14.8 (13.5 / 17.6 /
+// 14.8), 512 x 512 71 -> 6.0 (6.0 / 7.2 / 13.2), 2400 tokens 6144 x 2048 1293 -> 519 (521 / 497 /
+// 519; 116 of 157 TFLOP/s).
+template <int MODE> void blocks_f32(const GemmParams& p, int& rb, int& tb) {
+  const int cus = std::max(device_cus(), 1);
+  const double slices = ceil_div(p.K, S_ROW / 4);
+  double least = 0;
+  for (int r = MODE == kGated ? 2 : 1; r <= 4; r *= 2)
+    for (int t = 1; t <= 4; ++t) {
+      const int64_t wgs = (int64_t)ceil_div(p.N, (MODE == kGated ? r / 2 : r) * 16) * ceil_div(p.M, t * 16);
+      const double us = (double)((wgs + cus - 1) / cus) *
+                        (2.0 + slices * 0.036 * std::max(r * t, r + t));
+      if (least == 0 || us < least) rb = r, tb = t, least = us;
+    }
+}
+
+template <int MODE, int ACT>
+int launch_f32(const GemmParams& p, hipStream_t st) {
+  int rb = 4, tb = 4;
+  blocks_f32<MODE>(p, rb, tb);
+  CEA_REQUIRE(ceil_div(p.M, tb * 16) <= 65535, CEA_EUNSUPPORTED, "linear: %d rows exceed the f32 kernel's grid",
+              p.M);
+  if constexpr (MODE == kPlain)
+    if (rb == 1) return launch_tokens<float, MODE, ACT, 1>(p, tb, st);
+  if (rb == 2) return launch_tokens<float, MODE, ACT, 2>(p, tb, st);
+  return launch_tokens<float, MODE, ACT, 4>(p, tb, st);
+}
+
 template <typename T, int MODE, int ACT>
 int launch_act(const GemmParams& p, hipStream_t st) {
-  const int rb = weight_blocks<MODE>(p);
+  if constexpr (sizeof(T) == 4) return launch_f32<MODE, ACT>(p, st);
+  const int rb = weight_blocks<MODE>(p), tb = ceil_div(p.M, 16);
   if constexpr (MODE == kPlain)
-    if (rb == 1) return launch_blocks<T, MODE, ACT, 1>(p, st);
-  if (rb == 2) return launch_blocks<T, MODE, ACT, 2>(p, st);
-  return launch_blocks<T, MODE, ACT, 4>(p, st);
+    if (rb == 1) return launch_tokens<T, MODE, ACT, 1>(p, tb, st);
+  if (rb == 2) return launch_tokens<T, MODE, ACT, 2>(p, tb, st);
+  return launch_tokens<T, MODE, ACT, 4>(p, tb, st);
 }
 
 template <typename T>
@@ -228,7 +264,11 @@ int launch_typed(const GemmParams& p, int mode, int act, hipStream_t st) {
 }  // namespace
 
 int launch_linear_skinny(const GemmParams& p, int dtype, int mode, int act, hipStream_t st) {
-  return dtype == CEA_BF16 ? launch_typed<bf16>(p, mode, act, st) : launch_typed<f16>(p, mode, act, st);
+  switch (dtype) {
+    case CEA_BF16: return launch_typed<bf16>(p, mode, act, st);
+    case CEA_F16: return launch_typed<f16>(p, mode, act, st);
+    default: return launch_typed<float>(p, mode, act, st);
+  }
 }
 
 }  // namespace cea

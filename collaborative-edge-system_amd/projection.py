@@ -2,10 +2,10 @@
 drop-in for collab_infer/parallel/tensor_parallel.py:264-320 (``FusedColumnParallelLinear``)
 and the gate/up half of the gated MLP (collab_infer/models/llama.py:298-316).
 
-Both run on this package's gfx950 GEMM (csrc/gemm.hip): bf16 / f16 on the matrix cores with
-f32 accumulation rounded once to the input dtype, f32 / f64 (and shapes the matrix-core
-kernel does not take: K or a row stride not a multiple of 8, misaligned rows) on a generic
-kernel.
+Both run on this package's gfx950 GEMM (csrc/gemm.hip, csrc/gemm_skinny.hip): bf16 / f16 / f32
+on the matrix cores with f32 accumulation rounded once to the input dtype; f64, and shapes the
+matrix-core kernels do not take (K or a row stride not a multiple of 16 bytes, misaligned
+rows), on a generic kernel.
 
 * :func:`linear` - ``F.linear(x, weight, bias)`` for device tensors
 * :func:`fused_linear` - the same, returned as the per-projection column views of

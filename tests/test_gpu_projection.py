@@ -327,3 +327,23 @@ def test_linear_tile_heights_and_splits(cea, dev, dtype, m, k, n):
     torch.cuda.synchronize()
     assert rc == 0, nat.last_error()
     _check_linear(u, x, w, b, f"tiles without scratch {m}x{k}x{n} {dtype}")
+
+
+@pytest.mark.parametrize("m,k,n", [
+    (1, 4, 16),       # one 16-byte K group
+    (70, 36, 19),     # N not a multiple of 4, a K tail in the second slice
+    (200, 132, 1030), # several token blocks in the grid
+    (513, 516, 40),
+])
+def test_linear_f32_matrix_cores(cea, dev, m, k, n):
+    """f32 operands on the matrix cores at ragged sizes, plain (every element within the f32
+    accumulation bound) and gated (the unfused chain)."""
+    g = torch.Generator().manual_seed(m + 3 * k + n)
+    x, w, b = _operands(g, m, k, 2 * n, torch.float32)
+    xd, wd, bd = x.to(dev), w.to(dev), b.to(dev)
+    y = cea.projection.linear(xd, wd, bd)
+    act = cea.projection.linear_gated(xd, wd[:n], wd[n:], bd[:n], bd[n:], "silu")
+    chain = cea.layers.gated_mul(y[:, :n], y[:, n:], "silu")
+    torch.cuda.synchronize()
+    _check_linear(y, x, w, b, f"f32 {m}x{k}x{n}")
+    _same_as_chain(act, chain, f"f32 gated {m}x{k}x{n}")
