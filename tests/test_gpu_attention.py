@@ -372,3 +372,20 @@ def test_decode_with_more_rows_per_kv_head_than_a_unit(cea, dev, shape):
     torch.cuda.synchronize()
     assert_attention_close(out, lse, ro, rl, torch.bfloat16, str(shape))
     assert (plain.cpu().double() - ro.double()).abs().max().item() <= 2e-2
+
+
+@pytest.mark.parametrize("shape", [
+    (2, 300, 8, 4),    # KV heads of all rows a multiple of 8: dealt to the XCDs in turn
+    (1, 520, 16, 8),   # the same, two query heads per KV head, a short last query block
+    (4, 258, 6, 3),    # query heads of all rows a multiple of 8 only
+    (1, 270, 6, 2),    # neither
+], ids=str)
+def test_query_block_order(cea, dev, shape):
+    """Every (row, head, query block) is computed once whichever way the blocks are dealt."""
+    B, S, Hq, Hkv = shape
+    case = Case(B, S, S, Hq, Hkv, 64, "right_pad", True, seed=B + S)
+    q, k, v, qp, kp = case.tensors(torch.bfloat16)
+    out, lse = cea.attention_with_lse(q.to(dev), k.to(dev), v.to(dev), qp.to(dev), kp.to(dev))
+    ro, rl = ref.attention_with_lse(q, k, v, qp, kp, route="flash")
+    torch.cuda.synchronize()
+    assert_attention_close(out, lse, ro, rl, torch.bfloat16, str(case))
