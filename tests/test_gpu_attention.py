@@ -389,3 +389,22 @@ def test_query_block_order(cea, dev, shape):
     ro, rl = ref.attention_with_lse(q, k, v, qp, kp, route="flash")
     torch.cuda.synchronize()
     assert_attention_close(out, lse, ro, rl, torch.bfloat16, str(case))
+
+
+@pytest.mark.parametrize("rows,keys,first", [(1, 131, 0), (3, 67, 0), (2, 129, 1), (1, 64, 3)])
+def test_key_positions_at_any_offset(cea, dev, rows, keys, first):
+    """Odd key counts and blocks that begin at an odd slot of a larger position buffer (rows of
+    8-byte aligned positions) give what their 16-byte aligned copies give, bit for bit."""
+    case = Case(rows, 80, keys, 4, 2, 128, "random", True, seed=rows + keys)
+    q, k, v, qp, kp = (t.to(dev) for t in case.tensors(torch.bfloat16))
+    wide = torch.zeros(rows, (keys + 1) // 2 * 2, dtype=torch.int64, device=dev)
+    aligned = wide[:, :keys]
+    aligned.copy_(kp)
+    ro, rl = cea.attention_with_lse(q, k, v, qp, aligned)
+    buf = torch.full((rows, first + keys), 0, dtype=torch.int64, device=dev)
+    buf[:, first:] = kp
+    out, lse = cea.attention_with_lse(q, k, v, qp, buf[:, first:])
+    co, cl = ref.attention_with_lse(*(t.cpu() for t in (q, k, v, qp, kp)), route="flash")
+    torch.cuda.synchronize()
+    assert torch.equal(out, ro) and torch.equal(lse, rl)
+    assert_attention_close(out, lse, co, cl, torch.bfloat16, str(case))
