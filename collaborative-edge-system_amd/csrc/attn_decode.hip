@@ -4,7 +4,7 @@
 // is a few tokens, and the per-device compute of distributed_kv_attention
 // (collab_infer/parallel/sequence_parallel.py:250-280): every KV partition's partial
 // (out, lse) and their exact merge (merge_attention_list, attention.py:253-264), all on one
-// device and in three launches.
+// device and in two launches.
 //
 // HBM-bound design:
 //   * work item = (batch, kv head, one or two consecutive key chunks of one partition); the
@@ -18,12 +18,14 @@
 //     is refilled as soon as its fragments are in registers, so two tiles stay in flight; V is
 //     read back transposed with ds_read_b64_tr_b16; both tiles are XOR-swizzled so the
 //     fragment and transpose reads are free of LDS bank conflicts; the query rows come in by
-//     LDS-DMA as well, together with the item's tile masks;
-//   * a prepass reads the key positions once per batch row (not once per kv head) and turns
-//     them into a 16-bit visibility word per key (bit s: query s sees it) and a mask of the
-//     16-key tiles of each chunk that hold a visible key; the split kernel loads each tile's
-//     words with its K and V, never loads an invisible tile, and an item with empty masks
-//     writes nothing;
+//     LDS-DMA as well, in flight together with the key positions;
+//   * a workgroup first turns its item's key positions into a 16-bit visibility word per key
+//     (bit s: query s sees it) and a mask of the 16-key tiles that hold a visible key, both in
+//     LDS; it never loads an invisible tile, and an item without one writes only its (m, l) =
+//     (-inf, 0).  Every KV head's workgroups read the positions again (8 bytes a key, out of
+//     the caches, against 256 to 512 bytes of K and V); a prepass that did it once per batch row
+//     cost a launch and a round trip (one token of 8 sequences of 4096 keys, 32/4 heads of 64:
+//     17.7 us with it, 15.3 without);
 //   * the waves of a workgroup merge their online-softmax partials in LDS and write one
 //     (o unnormalised, m, l) partial per item with non-temporal stores (stores during the
 //     K/V stream cost its read rate far more than their size, so there are as few partial
@@ -40,13 +42,7 @@ namespace {
 constexpr int DTHREADS = 256;
 constexpr int NW = DTHREADS / 64;     // waves per workgroup
 constexpr int TK = 16;                // keys per tile
-#ifndef CEA_DECODE_CHMAX
-#define CEA_DECODE_CHMAX 1024
-#endif
-#ifndef CEA_DECODE_ITEMS
-#define CEA_DECODE_ITEMS 8192
-#endif
-constexpr int CHMAX = CEA_DECODE_CHMAX;  // keys per chunk at most
+constexpr int CHMAX = 1024;           // keys per chunk at most
 static_assert(CHMAX % DTHREADS == 0 && CHMAX <= 4 * DTHREADS, "one 64-bit tile mask per chunk");
 constexpr float kRescaleLog2 = 8.0f;  // lazy-rescale threshold, log2 units
 
@@ -97,8 +93,7 @@ template <> struct Mfma16<f16> {
 template <int D> struct DLayout {
   static constexpr int ROW = D * 2;                 // bytes per key row
   static constexpr int TILE_BYTES = TK * ROW;       // one K or V tile
-  static constexpr int VIS_OFF = 2 * TILE_BYTES;    // 16 visibility words after K and V
-  static constexpr int BUF_BYTES = VIS_OFF + 64;
+  static constexpr int BUF_BYTES = 2 * TILE_BYTES;
   static constexpr int WAVE_BYTES = 2 * BUF_BYTES;  // double-buffered per wave
   static constexpr int LDS_BYTES = NW * WAVE_BYTES;
   static constexpr int LOADS = TILE_BYTES / 1024;   // direct loads per tensor per tile
@@ -180,52 +175,6 @@ __device__ __forceinline__ int items_of_row(const DecodeParams& p, int b) {
   return b < p.pair_rows ? p.item_begin[p.nparts] : p.chunk_begin[p.nparts];
 }
 
-// Visibility prepass, one workgroup per (chunk, batch): for every key of the chunk a word whose
-// bit s says whether query s of the batch sees it (k_pos >= 0 and, when causal,
-// k_pos <= q_pos[s]), and for the chunk a mask of the 16-key tiles holding a visible key.
-// The split kernel then never reads positions, and skips invisible tiles without loading them.
-__global__ __launch_bounds__(DTHREADS) void decode_vis_kernel(const DecodeParams p) {
-  const int chunk = blockIdx.x, b = blockIdx.y;
-  const int part = part_of(p, chunk);
-  const int key0 = (chunk - p.chunk_begin[part]) * p.chunk;
-  const int nkeys = min(p.chunk, p.Sk[part] - key0);
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int total_chunks = p.chunk_begin[p.nparts];
-  __shared__ uint32_t wmask[NW];
-  // every load is issued before the first wait (key indices clamped into the chunk)
-  const int64_t* kp = p.k_pos[part] + b * p.kps[part][0];
-  const int64_t kps = p.kps[part][1];
-  int64_t pk[4];
-#pragma unroll
-  for (int u = 0; u < 4; ++u) pk[u] = kp[(int64_t)(key0 + min(tid * 4 + u, nkeys - 1)) * kps];
-  uint32_t words[4] = {0u, 0u, 0u, 0u};
-  for (int q = 0; q < p.Sq; ++q) {
-    const int64_t qs = p.q_pos[b * p.qps_b + (int64_t)q * p.qps_s];
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-      if (tid * 4 + u < nkeys && pk[u] >= 0 && (!p.causal || pk[u] <= qs)) words[u] |= 1u << q;
-  }
-  if (tid * 4 < p.chunk) {
-    uint2 packed = {words[0] | (words[1] << 16), words[2] | (words[3] << 16)};
-    *(uint2*)(p.vis + ((int64_t)b * total_chunks + chunk) * p.chunk + tid * 4) = packed;
-  }
-  // lanes 4j..4j+3 of wave w hold tile w*16 + j
-  const uint64_t bal = __ballot((words[0] | words[1] | words[2] | words[3]) != 0);
-  if (lane == 0) {
-    uint32_t m = 0;
-#pragma unroll
-    for (int j = 0; j < 16; ++j) m |= (((bal >> (4 * j)) & 0xfu) != 0 ? 1u : 0u) << j;
-    wmask[wave] = m;
-  }
-  __syncthreads();
-  if (tid == 0) {
-    uint64_t m = 0;
-#pragma unroll
-    for (int w = 0; w < NW; ++w) m |= (uint64_t)wmask[w] << (16 * w);
-    p.tile_mask[(int64_t)b * total_chunks + chunk] = m;
-  }
-}
-
 // Partial layout: [B][Hkv][total_chunks][NR][D + 2] floats: o (relative to m), m, l, where
 // m is in natural-log units (max of scale*q.k) and l = sum exp(scale*q.k - m).
 template <typename T, int D, int NR>
@@ -235,6 +184,8 @@ __global__ __launch_bounds__(DTHREADS, 2) void decode_split_kernel(const DecodeP
   extern __shared__ __attribute__((aligned(16))) char dsmem[];
   __shared__ float red_m[NW][NR];
   __shared__ float red_l[NW][NR];
+  __shared__ __attribute__((aligned(16))) uint16_t vis_s[2 * CHMAX];   // words of the item's chunks
+  __shared__ uint64_t wmask[2][NW];
 
   // 1-D grid: pair items of rows [0, pair_rows), then single-chunk items of the other rows;
   // item fastest, then unit, then batch row - except when several units read one KV head
@@ -270,7 +221,7 @@ __global__ __launch_bounds__(DTHREADS, 2) void decode_split_kernel(const DecodeP
   char* wb = dsmem + wave * L::WAVE_BYTES;
 
   // ---- the query rows r = s * G + g of this kv head come straight into the wave's first tile
-  // buffer (free until the first tile load), in flight together with the chunk's tile mask, so
+  // buffer (free until the first tile load), in flight together with the key positions, so
   // the workgroup starts streaming after one memory round trip
   {
     constexpr int QROWS = 1024 / L::ROW;  // query rows one 1 KB load covers
@@ -286,13 +237,62 @@ __global__ __launch_bounds__(DTHREADS, 2) void decode_split_kernel(const DecodeP
       buffer_load_lds16(qrs, wb + i * 1024, off);
     }
   }
-  const uint64_t mask = p.tile_mask[(int64_t)b * total_chunks + chunk];
-  const uint64_t mask1 = nch > 1 ? p.tile_mask[(int64_t)b * total_chunks + chunk + 1] : 0ull;
-  wait_vmcnt<0>();  // query rows in LDS (also before an early exit frees the LDS)
-  // no key of the item is visible to any query row: no partial (the reduction reads the masks)
-  if ((mask | mask1) == 0) return;
   const int Sk = p.Sk[part];
   const int key0 = (chunk - p.chunk_begin[part]) * p.chunk;
+
+  // ---- visibility of the item's keys: thread t takes keys t, t + 256, ... of each chunk, so 16
+  // lanes hold one tile; every load is issued before the first wait (indices clamped)
+  {
+    constexpr int PER = CHMAX / DTHREADS;
+    const int64_t* kp = p.k_pos[part] + b * p.kps[part][0];
+    const int64_t kps = p.kps[part][1];
+    int64_t pk[2][PER];
+#pragma unroll
+    for (int ch = 0; ch < 2; ++ch)
+#pragma unroll
+      for (int u = 0; u < PER; ++u) {
+        pk[ch][u] = -1;
+        if (ch < nch && u * DTHREADS < p.chunk)
+          pk[ch][u] = kp[(int64_t)min(key0 + ch * p.chunk + u * DTHREADS + tid, Sk - 1) * kps];
+      }
+#pragma unroll
+    for (int ch = 0; ch < 2; ++ch) {
+      uint64_t m = 0;
+      if (ch < nch) {
+        const int nkeys = min(p.chunk, Sk - key0 - ch * p.chunk);
+        uint32_t words[PER] = {};
+        for (int q = 0; q < p.Sq; ++q) {
+          const int64_t qs = p.q_pos[b * p.qps_b + (int64_t)q * p.qps_s];
+#pragma unroll
+          for (int u = 0; u < PER; ++u)
+            if (u * DTHREADS + tid < nkeys && pk[ch][u] >= 0 && (!p.causal || pk[ch][u] <= qs))
+              words[u] |= 1u << q;
+        }
+#pragma unroll
+        for (int u = 0; u < PER; ++u) {
+          if (u * DTHREADS + tid < p.chunk) vis_s[ch * CHMAX + u * DTHREADS + tid] = (uint16_t)words[u];
+          const uint64_t bal = __ballot(words[u] != 0);
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            if ((bal >> (16 * j)) & 0xffffu) m |= 1ull << (u * (DTHREADS / TK) + wave * 4 + j);
+        }
+      }
+      if (lane == 0) wmask[ch][wave] = m;
+    }
+  }
+  wait_vmcnt<0>();  // query rows in LDS (also before an early exit frees the LDS)
+  __syncthreads();
+  uint64_t mask = 0, mask1 = 0;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) mask |= wmask[0][w], mask1 |= wmask[1][w];
+  // no key of the item is visible to any query row: the partial is (m, l) alone
+  if ((mask | mask1) == 0) {
+    if (tid < NR) {
+      part_out[tid * (D + 2) + D] = -__builtin_inff();
+      part_out[tid * (D + 2) + D + 1] = 0.f;
+    }
+    return;
+  }
 
   // ---- this lane's Q fragments (B operand of S = K.Q^T), sign folded for a negative scale
   const float scale = (float)p.scale;
@@ -316,7 +316,6 @@ __global__ __launch_bounds__(DTHREADS, 2) void decode_split_kernel(const DecodeP
   // ---- per-lane constant offsets
   const char* kbase = (const char*)((const T*)p.k[part] + b * p.ks[part][0] + kvh * p.ks[part][2]);
   const char* vbase = (const char*)((const T*)p.v[part] + b * p.vs[part][0] + kvh * p.vs[part][2]);
-  const char* visbase = (const char*)(p.vis + ((int64_t)b * total_chunks + chunk) * p.chunk);
   const uint32_t krow = (uint32_t)(p.ks[part][1] * sizeof(T)), vrow = (uint32_t)(p.vs[part][1] * sizeof(T));
   uint32_t k_voff[L::LOADS], v_voff[L::LOADS];
 #pragma unroll
@@ -366,12 +365,8 @@ __global__ __launch_bounds__(DTHREADS, 2) void decode_split_kernel(const DecodeP
     for (int i = 0; i < L::LOADS; ++i) buffer_load_lds16_nt(krs, kb + i * 1024, k_voff[i]);
 #pragma unroll
     for (int i = 0; i < L::LOADS; ++i) buffer_load_lds16_nt(vrs, kb + L::TILE_BYTES + i * 1024, v_voff[i]);
-    if (lane < TK * 2 / 4) {  // 16 visibility words, 4 bytes per lane
-      const i32x4 wrs = make_rsrc(visbase + t * TK * 2, TK * 2);
-      buffer_load_lds4(wrs, kb + L::VIS_OFF, lane * 4);
-    }
   };
-  constexpr int LOADS_PER_TILE = 2 * L::LOADS + 1;
+  constexpr int LOADS_PER_TILE = 2 * L::LOADS;
 
   f32x4 o[D / 16];
 #pragma unroll
@@ -384,11 +379,12 @@ __global__ __launch_bounds__(DTHREADS, 2) void decode_split_kernel(const DecodeP
     s16x4 v[D / 16];
     uint2 vis;
   };
-  auto read_frags = [&](int buf, Frags& f) {
+  auto read_frags = [&](int buf, int t, Frags& f) {
     const char* kb = wb + buf * L::BUF_BYTES;
 #pragma unroll
     for (int ks = 0; ks < D / 32; ++ks) f.k[ks] = *(const frag8*)(kb + k_raddr[ks]);
-    f.vis = *(const uint2*)(kb + L::VIS_OFF + grp * 8);  // keys grp*4 .. grp*4+3
+    const int k0 = t < tpc ? t * TK : CHMAX + (t - tpc) * TK;
+    f.vis = *(const uint2*)(vis_s + k0 + grp * 4);  // keys grp*4 .. grp*4+3
 #pragma unroll
     for (int dt = 0; dt < D / 16; ++dt)
       f.v[dt] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(kb + v_raddr[dt]));
@@ -439,7 +435,7 @@ __global__ __launch_bounds__(DTHREADS, 2) void decode_split_kernel(const DecodeP
       else
         wait_vmcnt<0>();
       Frags f;
-      read_frags(buf, f);
+      read_frags(buf, t, f);
       const int t2 = pop_tile();
       if (t2 >= 0) {
         wait_lgkmcnt0();  // fragments in registers before the buffer is refilled
@@ -556,14 +552,9 @@ __global__ __launch_bounds__(RTHREADS) void decode_reduce_kernel(const DecodePar
     const int j = wave + RWAVES * k;
     pre[k] = total > 0 ? RV::load(base + (j < total ? j : 0) * cstride + FPL * lane) : V{};
   }
-  // items without a visible key wrote no partial: their weight is 0
-  const uint64_t* cmask = p.tile_mask + (int64_t)b * total_chunks;
-  auto item_ml = [&](int j) -> float2 {  // (m, l) of item j, (-inf, 0) for an empty item
-    const DecodeItem it = item_of(p, b, j);
-    const bool live = (cmask[it.chunk] | (it.nch > 1 ? cmask[it.chunk + 1] : 0ull)) != 0;
-    const float2 ml = *(const float2*)(base + j * cstride + D);
-    return live ? ml : make_float2(-__builtin_inff(), 0.f);
-  };
+  // (m, l) of item j; an item without a visible key wrote (-inf, 0) and no output: its weight
+  // is 0 and what the partial holds is not used
+  auto item_ml = [&](int j) -> float2 { return *(const float2*)(base + j * cstride + D); };
   // lse = logsumexp over the partitions' lse_p (the reference merge's formula)
   auto combine = [&](const float (&lp)[CEA_MAX_PARTS]) -> float {
     if (p.nparts == 1) return lp[0];
@@ -707,8 +698,6 @@ template <typename T, int D, int NR>
 int launch_nr(const DecodeParams& p, hipStream_t st) {
   const int total = p.chunk_begin[p.nparts];
   if (total > 0) {
-    hipLaunchKernelGGL(decode_vis_kernel, dim3(total, p.B), dim3(DTHREADS), 0, st, p);
-    CEA_CHECK_LAUNCH("decode_vis");
     const hipError_t e = reserve_lds<decode_split_kernel<T, D, NR>>(DLayout<D>::LDS_BYTES);
     CEA_REQUIRE(e == hipSuccess, CEA_ELAUNCH, "decode: cannot reserve %d bytes of LDS: %s",
                 DLayout<D>::LDS_BYTES, hipGetErrorString(e));
@@ -771,15 +760,22 @@ bool decode_supported(int32_t Sq, int32_t Hq, int32_t Hkv, int32_t D, int32_t dt
   return Hq <= CEA_MAX_MAPPED_HEADS && decode_rows(Sq, 1) != 0;
 }
 
-// Work items wanted per launch: enough to fill 256 CUs several times.  An item's bytes per key
+// Work items a launch needs before its chunks grow past 256 keys: about two rounds of resident
+// workgroups (two per compute unit), since an item's start (positions, then its first tiles) is
+// hidden only behind the other resident item, and longer items have fewer of them.  Measured
+// (us, targets 8192 / 2048 / 1024; 32/8 heads, D = 128): 16 rows of 8000 keys 105 / 93 / 93, 32
+// of 4000 93 / 79 / 77, 8 of 32000 in two partitions 141 / 122 / 122.  An item's bytes per key
 // scale with the head size, so the count scales with it too (a head size of 64 takes half as
 // many, twice the keys each: the same bytes per item as at 128).
-static int64_t decode_item_target(int32_t D) { return (int64_t)CEA_DECODE_ITEMS * D / 128; }
+static int64_t decode_item_target(int32_t D) { return (int64_t)1024 * D / 128; }
 
 int decode_plan_chunk(int64_t keys_per_head, int32_t B, int32_t units, int32_t D) {
-  // chunks of 256..1024 keys
+  // 64 keys (one tile per wave) up to 256 while the items are fewer than the compute units, so a
+  // short cache is read by all of them in one or two tiles each (one sequence of 300 keys, 8 KV
+  // heads: 12.3 us with 64-key chunks, 14.1 with 256); then 256..1024 by the item target
   const int64_t heads = (int64_t)B * units;
-  int ch = 256;
+  int ch = 64;
+  while (ch < 256 && heads * ((keys_per_head + ch - 1) / ch) > 256) ch *= 2;
   while (ch < CHMAX && heads * ((keys_per_head + ch - 1) / ch) > decode_item_target(D)) ch *= 2;
   return ch;
 }

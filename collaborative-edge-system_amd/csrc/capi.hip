@@ -156,8 +156,7 @@ struct DecodePlan {
   int chunk;
   int total_chunks;
   int nr;
-  size_t partial_bytes;  // partials + visibility words + tile masks
-  size_t vis_offset, mask_offset;
+  size_t partial_bytes;
 };
 
 // Work units of the decode kernels: G consecutive query heads that read one KV head, whose
@@ -180,8 +179,8 @@ static DecodeUnits decode_units(int64_t Hq, int64_t Hkv, int64_t Sq, const HeadM
   return {(int32_t)Hq, 1, 1};
 }
 
-// A plan the decode launches can take: at most kDecodeMaxChunks chunks per batch row, batch
-// rows within the visibility pass's second grid dimension, and every grid within 31 bits
+// A plan the decode launches can take: at most kDecodeMaxChunks chunks per batch row, fewer
+// than 65536 batch rows, and every grid within 31 bits
 // (the split kernel's: one work item per unit and chunk at most, before chunk pairs halve
 // it; the reduction's: one workgroup per output row).
 static bool decode_plan_fits(int64_t B, int64_t Sq, int64_t Hq, int64_t units,
@@ -199,10 +198,8 @@ static DecodePlan plan_decode(const int64_t* Sk, int n, int64_t B, int64_t Sq, i
   pl.total_chunks = 0;
   for (int i = 0; i < n; ++i) pl.total_chunks += (int)((Sk[i] + pl.chunk - 1) / pl.chunk);
   pl.nr = decode_rows((int32_t)Sq, (int32_t)G);
-  pl.vis_offset = align_up((size_t)(B * units) * pl.total_chunks * (pl.nr > 0 ? pl.nr : 1) *
-                               (D + 2) * sizeof(float), 256);
-  pl.mask_offset = pl.vis_offset + align_up((size_t)B * pl.total_chunks * pl.chunk * sizeof(uint16_t), 256);
-  pl.partial_bytes = pl.mask_offset + align_up((size_t)B * pl.total_chunks * sizeof(uint64_t), 256);
+  pl.partial_bytes = align_up((size_t)(B * units) * pl.total_chunks * (pl.nr > 0 ? pl.nr : 1) *
+                                  (D + 2) * sizeof(float), 256);
   return pl;
 }
 
@@ -269,8 +266,6 @@ static int run_decode(const AttnParams* blocks, int n, cea_tensor* part_out, cea
   d.in_dtype = a.in_dtype;
   d.map = a.map;
   d.partial = (float*)ws;
-  d.vis = (uint16_t*)(ws + pl.vis_offset);
-  d.tile_mask = (uint64_t*)(ws + pl.mask_offset);
   d.G = du.G;
   d.units = du.units;
   d.per_head = du.per_head;

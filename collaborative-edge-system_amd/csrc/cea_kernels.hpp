@@ -106,11 +106,8 @@ struct DecodeParams {
   int32_t in_dtype;
   HeadMap map;
   // partial results [B, units, total_chunks, NR rows (s, g)] x {D + 2} floats (o unnormalised,
-  // m, l); per-key visibility words [B, total_chunks, chunk] (bit s: query s sees the key);
-  // per-chunk masks [B, total_chunks] of 16-key tiles with a visible key
+  // m, l)
   float* partial;
-  uint16_t* vis;
-  uint64_t* tile_mask;
   int32_t G;                 // query heads of one work unit (all read one KV head)
   // work units per batch row: unit u holds query heads u*G .. u*G+G-1 and reads KV head
   // map.kv_of(u*G) - a KV head's whole group, part of it, or (G = 1) one query head of an

@@ -408,3 +408,31 @@ def test_key_positions_at_any_offset(cea, dev, rows, keys, first):
     torch.cuda.synchronize()
     assert torch.equal(out, ro) and torch.equal(lse, rl)
     assert_attention_close(out, lse, co, cl, torch.bfloat16, str(case))
+
+
+@pytest.mark.parametrize("batch,queries,keys,hkv", [
+    (1, 1, 1, 1),       # one key
+    (1, 2, 65, 2),      # one key past a 64-key chunk
+    (2, 3, 300, 4),     # 64-key chunks, a short last one
+    (1, 1, 2049, 8),    # 128-key chunks
+    (5, 1, 1500, 8),    # 256-key chunks
+    (40, 1, 1030, 8),   # 1024-key chunks, the second of 6 keys
+])
+@pytest.mark.parametrize("d", [64, 128])
+def test_decode_chunks(cea, dev, batch, queries, keys, hkv, d):
+    """Every chunk size of the split-KV decode, with rows of which most chunks hold no visible
+    key (they write no output partial) and a row without any."""
+    g = torch.Generator().manual_seed(batch + keys)
+    q = torch.randn(batch, queries, 4 * hkv, d, generator=g).to(torch.bfloat16)
+    k = torch.randn(batch, keys, hkv, d, generator=g).to(torch.bfloat16)
+    v = torch.randn(batch, keys, hkv, d, generator=g).to(torch.bfloat16)
+    kp = torch.arange(keys).repeat(batch, 1)
+    kp[0, keys // 8 + 1:] = -1
+    kp[-1, : keys // 2] = -1
+    if batch > 2:
+        kp[1] = -1
+    qp = torch.arange(keys - queries, keys).clamp(min=0).repeat(batch, 1)
+    out, lse = cea.attention_with_lse(*(t.to(dev) for t in (q, k, v, qp, kp)))
+    ro, rl = ref.attention_with_lse(q, k, v, qp, kp, route="flash")
+    torch.cuda.synchronize()
+    assert_attention_close(out, lse, ro, rl, torch.bfloat16, f"decode {batch}x{queries}x{keys}")
