@@ -324,10 +324,14 @@ def distributed_kv_attention(
 
     Every rank's partition runs in one split-KV launch, the exact merge in its reduction;
     :func:`distributed_kv_attention_packed` runs the multi-device message flow instead."""
+    if comm.size == 1 and k_local.shape[1] and q.shape[1]:
+        # one partition: the kernels write q.dtype themselves (the same rounding of the same
+        # f32 result, without a cast pass and the lse)
+        return attention(q, k_local, v_local, q_pos, k_pos_local, causal=causal, scale=scale,
+                         kv_map=kv_map, kv_block=kv_block)
     if comm.size == 1:
-        o, _ = attention_with_lse(q, k_local, v_local, q_pos, k_pos_local, causal=causal,
-                                  scale=scale, kv_map=kv_map, kv_block=kv_block)
-        return o.to(q.dtype)
+        return attention_with_lse(q, k_local, v_local, q_pos, k_pos_local, causal=causal, scale=scale,
+                                  kv_map=kv_map, kv_block=kv_block)[0].to(q.dtype)
     parts = _dkv_partitions(comm, (k_local, v_local, k_pos_local))
     if kv_block is not None:
         partial = [attention_with_lse(q, kk, vv, q_pos, pp, causal=causal, scale=scale,

@@ -366,3 +366,20 @@ def test_distributed_kv_more_ranks_than_one_launch(cea, dev, nranks):
     assert_attention_close(o2, l2, ro.float(), rl, torch.bfloat16, f"{nranks} ranks merged")
     for i, ((po, pl), (qo, ql)) in enumerate(zip(per, rparts)):
         assert_attention_close(po, pl, qo, ql, torch.bfloat16, f"rank {i} partial")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("queries,keys", [(1, 300), (40, 2000), (2, 0)])
+def test_one_partition_writes_the_query_dtype(cea, dev, dtype, queries, keys):
+    """A group of one returns the f32 result cast to the query dtype, bit for bit, on the decode
+    route, the key-split prefill route and for an empty cache."""
+    g = torch.Generator().manual_seed(queries + keys)
+    q = torch.randn(2, queries, 8, 64, generator=g).to(dtype).to(dev)
+    k = torch.randn(2, keys, 2, 64, generator=g).to(dtype).to(dev)
+    v = torch.randn(2, keys, 2, 64, generator=g).to(dtype).to(dev)
+    qp = torch.arange(keys, keys + queries, device=dev).repeat(2, 1)
+    kp = torch.arange(keys, device=dev).repeat(2, 1)
+    got = cea.distributed_kv_attention(q, k, v, qp, kp, cea.LocalGroup(1, 0))
+    want = cea.attention_with_lse(q, k, v, qp, kp)[0].to(dtype)
+    torch.cuda.synchronize()
+    assert got.dtype == dtype and torch.equal(got, want)
