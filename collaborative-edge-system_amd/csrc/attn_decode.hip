@@ -143,9 +143,10 @@ __device__ __forceinline__ float wave_sum_lanes(float v) {
 }
 #undef CEA_DPP_F32
 
-__device__ __forceinline__ int part_of(const DecodeParams& p, int chunk) {
+template <class P> __device__ __forceinline__ int part_of(const P& p, int chunk) {
   int part = 0;
-  while (part + 1 < p.nparts && chunk >= p.chunk_begin[part + 1]) ++part;
+  if constexpr (P::kParts > 1)
+    while (part + 1 < p.nparts && chunk >= p.chunk_begin[part + 1]) ++part;
   return part;
 }
 
@@ -156,11 +157,12 @@ __device__ __forceinline__ int part_of(const DecodeParams& p, int chunk) {
 struct DecodeItem {
   int part, chunk, nch;
 };
-__device__ __forceinline__ DecodeItem item_of(const DecodeParams& p, int b, int item) {
+template <class P> __device__ __forceinline__ DecodeItem item_of(const P& p, int b, int item) {
   DecodeItem it;
   if (b < p.pair_rows) {
     int part = 0;
-    while (part + 1 < p.nparts && item >= p.item_begin[part + 1]) ++part;
+    if constexpr (P::kParts > 1)
+      while (part + 1 < p.nparts && item >= p.item_begin[part + 1]) ++part;
     it.part = part;
     it.chunk = p.chunk_begin[part] + 2 * (item - p.item_begin[part]);
     it.nch = min(2, p.chunk_begin[part + 1] - it.chunk);
@@ -171,14 +173,18 @@ __device__ __forceinline__ DecodeItem item_of(const DecodeParams& p, int b, int 
   }
   return it;
 }
-__device__ __forceinline__ int items_of_row(const DecodeParams& p, int b) {
-  return b < p.pair_rows ? p.item_begin[p.nparts] : p.chunk_begin[p.nparts];
+// partitions of the call
+template <class P> __device__ __forceinline__ int parts_of(const P& p) {
+  return P::kParts == 1 ? 1 : p.nparts;
+}
+template <class P> __device__ __forceinline__ int items_of_row(const P& p, int b) {
+  return b < p.pair_rows ? p.item_begin[parts_of(p)] : p.chunk_begin[parts_of(p)];
 }
 
 // Partial layout: [B][Hkv][total_chunks][NR][D + 2] floats: o (relative to m), m, l, where
 // m is in natural-log units (max of scale*q.k) and l = sum exp(scale*q.k - m).
-template <typename T, int D, int NR>
-__global__ __launch_bounds__(DTHREADS, 2) void decode_split_kernel(const DecodeParams p) {
+template <typename T, int D, int NR, class P>
+__global__ __launch_bounds__(DTHREADS, 2) void decode_split_kernel(const P p) {
   typedef DLayout<D> L;
   typedef typename Mfma16<T>::frag8 frag8;
   extern __shared__ __attribute__((aligned(16))) char dsmem[];
@@ -191,10 +197,11 @@ __global__ __launch_bounds__(DTHREADS, 2) void decode_split_kernel(const DecodeP
   // item fastest, then unit, then batch row - except when several units read one KV head
   // (per_head): units go fastest then, so those reading one KV head's chunk run side by side
   // and share its reads in the caches
-  const int total_chunks = p.chunk_begin[p.nparts];
+  const int nparts = parts_of(p);
+  const int total_chunks = p.chunk_begin[nparts];
   int b, unit, item;
   {
-    const int n2 = p.item_begin[p.nparts];
+    const int n2 = p.item_begin[nparts];
     const int first = p.pair_rows * p.units * n2;
     const int id = blockIdx.x;
     const int r = id < first ? id : id - first;
@@ -520,19 +527,20 @@ template <> struct RVec<64> {
   static __device__ __forceinline__ float get(V a, int) { return a; }
 };
 
-template <typename O, int D, int NR>
-__global__ __launch_bounds__(RTHREADS) void decode_reduce_kernel(const DecodeParams p) {
+template <typename O, int D, int NR, class P>
+__global__ __launch_bounds__(RTHREADS) void decode_reduce_kernel(const P p) {
   typedef RVec<D> RV;
   typedef typename RV::V V;
   constexpr int FPL = D / 64;  // output features per lane
   const int row = blockIdx.x;  // (b, s, h)
+  const int nparts = parts_of(p);
   const int h = row % p.Hq;
   const int s = (row / p.Hq) % p.Sq;
   const int b = row / (p.Hq * p.Sq);
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int unit = h / p.G;  // the work unit that computed this head
   const int r = s * p.G + (h - unit * p.G);
-  const int total_chunks = p.chunk_begin[p.nparts];
+  const int total_chunks = p.chunk_begin[nparts];
   const int total = items_of_row(p, b);  // work items (partials) of this batch row
   const int* ibegin = b < p.pair_rows ? p.item_begin : p.chunk_begin;
   const int64_t cstride = (int64_t)NR * (D + 2);
@@ -556,26 +564,26 @@ __global__ __launch_bounds__(RTHREADS) void decode_reduce_kernel(const DecodePar
   // is 0 and what the partial holds is not used
   auto item_ml = [&](int j) -> float2 { return *(const float2*)(base + j * cstride + D); };
   // lse = logsumexp over the partitions' lse_p (the reference merge's formula)
-  auto combine = [&](const float (&lp)[CEA_MAX_PARTS]) -> float {
-    if (p.nparts == 1) return lp[0];
+  auto combine = [&](const float (&lp)[P::kParts]) -> float {
+    if (nparts == 1) return lp[0];
     float mx = -__builtin_inff();
-    for (int part = 0; part < p.nparts; ++part) mx = fmaxf(mx, lp[part]);
+    for (int part = 0; part < nparts; ++part) mx = fmaxf(mx, lp[part]);
     const float shift = is_inf(mx) ? 0.f : mx;
     float sum = 0.f;
-    for (int part = 0; part < p.nparts; ++part) sum = add_rn(sum, expf(lp[part] - shift));
+    for (int part = 0; part < nparts; ++part) sum = add_rn(sum, expf(lp[part] - shift));
     return logf(sum) + shift;
   };
   // statistics in wave 0 alone (lane reductions, no workgroup barriers): per partition
   // M_p = max m, L_p = sum l * exp(m - M_p), lse_p = M_p + log L_p; then lse and the item
   // weights exp(m - lse)
-  __shared__ float s_lse[CEA_MAX_PARTS + 1];
-  float lp[CEA_MAX_PARTS];
+  __shared__ float s_lse[P::kParts + 1];
+  float lp[P::kParts];
   if (total <= 64) {
     // one item per lane: its (m, l) stays in registers from the load to the weight, and the
     // workgroup waits at one barrier (the weights) instead of two
     if (wave == 0) {
       const float2 ml = lane < total ? item_ml(lane) : make_float2(-__builtin_inff(), 0.f);
-      for (int part = 0; part < p.nparts; ++part) {
+      for (int part = 0; part < nparts; ++part) {
         const bool in = lane >= ibegin[part] && lane < ibegin[part + 1];
         const float mx = wave_max_lanes(in ? ml.x : -__builtin_inff());
         const bool use = in && mx != -__builtin_inff() && ml.x != -__builtin_inff();
@@ -586,8 +594,8 @@ __global__ __launch_bounds__(RTHREADS) void decode_reduce_kernel(const DecodePar
       const bool empty = lse == -__builtin_inff();
       if (lane < total) w_s[lane] = (empty || ml.x == -__builtin_inff()) ? 0.f : expf(ml.x - lse);
       if (lane == 0) {
-        for (int part = 0; part < p.nparts; ++part) s_lse[part] = lp[part];
-        s_lse[p.nparts] = lse;
+        for (int part = 0; part < nparts; ++part) s_lse[part] = lp[part];
+        s_lse[nparts] = lse;
       }
     }
   } else {
@@ -598,7 +606,7 @@ __global__ __launch_bounds__(RTHREADS) void decode_reduce_kernel(const DecodePar
     }
     __syncthreads();
     if (wave == 0) {
-      for (int part = 0; part < p.nparts; ++part) {
+      for (int part = 0; part < nparts; ++part) {
         const int c0 = ibegin[part], c1 = ibegin[part + 1];
         float mx = -__builtin_inff();
         for (int j = c0 + lane; j < c1; j += 64) mx = fmaxf(mx, m_s[j]);
@@ -615,15 +623,15 @@ __global__ __launch_bounds__(RTHREADS) void decode_reduce_kernel(const DecodePar
       for (int j = lane; j < total; j += 64)
         w_s[j] = (empty || m_s[j] == -__builtin_inff()) ? 0.f : expf(m_s[j] - lse);
       if (lane == 0) {
-        for (int part = 0; part < p.nparts; ++part) s_lse[part] = lp[part];
-        s_lse[p.nparts] = lse;
+        for (int part = 0; part < nparts; ++part) s_lse[part] = lp[part];
+        s_lse[nparts] = lse;
       }
     }
   }
   __syncthreads();
-  float lse_p[CEA_MAX_PARTS];
-  for (int part = 0; part < p.nparts; ++part) lse_p[part] = s_lse[part];
-  const float lse = s_lse[p.nparts];
+  float lse_p[P::kParts];
+  for (int part = 0; part < nparts; ++part) lse_p[part] = s_lse[part];
+  const float lse = s_lse[nparts];
 
   // weighted sum of the chunk outputs over [c0, c1): wave w takes chunks w, w + 4, ...; the
   // first RPF of them came in with the statistics (pre), later ones are read when their weight
@@ -655,7 +663,7 @@ __global__ __launch_bounds__(RTHREADS) void decode_reduce_kernel(const DecodePar
   V res;
   if (p.part_out[0]) {
     res = V{};
-    for (int part = 0; part < p.nparts; ++part) {
+    for (int part = 0; part < nparts; ++part) {
       const V t = chunk_sum(ibegin[part], ibegin[part + 1]);
       res = RV::add(res, t);
       if (wave == 0) {
@@ -694,15 +702,15 @@ __global__ __launch_bounds__(RTHREADS) void decode_reduce_kernel(const DecodePar
   }
 }
 
-template <typename T, int D, int NR>
-int launch_nr(const DecodeParams& p, hipStream_t st) {
+template <typename T, int D, int NR, class P>
+int launch_parts(const P& p, hipStream_t st) {
   const int total = p.chunk_begin[p.nparts];
   if (total > 0) {
-    const hipError_t e = reserve_lds<decode_split_kernel<T, D, NR>>(DLayout<D>::LDS_BYTES);
+    const hipError_t e = reserve_lds<decode_split_kernel<T, D, NR, P>>(DLayout<D>::LDS_BYTES);
     CEA_REQUIRE(e == hipSuccess, CEA_ELAUNCH, "decode: cannot reserve %d bytes of LDS: %s",
                 DLayout<D>::LDS_BYTES, hipGetErrorString(e));
     const int64_t grid = ((int64_t)p.pair_rows * p.item_begin[p.nparts] + (int64_t)(p.B - p.pair_rows) * total) * p.units;
-    hipLaunchKernelGGL((decode_split_kernel<T, D, NR>), dim3((unsigned)grid), dim3(DTHREADS),
+    hipLaunchKernelGGL((decode_split_kernel<T, D, NR, P>), dim3((unsigned)grid), dim3(DTHREADS),
                        DLayout<D>::LDS_BYTES, st, p);
     CEA_CHECK_LAUNCH("decode_split");
   }
@@ -711,22 +719,62 @@ int launch_nr(const DecodeParams& p, hipStream_t st) {
   const int stage = 2 * total * (int)sizeof(float);
   hipError_t e;
   if (p.out_dtype == CEA_F32) {
-    e = reserve_lds<decode_reduce_kernel<float, D, NR>>(2 * RCH * (int)sizeof(float));
+    e = reserve_lds<decode_reduce_kernel<float, D, NR, P>>(2 * RCH * (int)sizeof(float));
     if (e == hipSuccess)
-      hipLaunchKernelGGL((decode_reduce_kernel<float, D, NR>), dim3(rows), dim3(RTHREADS), stage, st, p);
+      hipLaunchKernelGGL((decode_reduce_kernel<float, D, NR, P>), dim3(rows), dim3(RTHREADS), stage, st, p);
   } else if (p.out_dtype == CEA_BF16) {
-    e = reserve_lds<decode_reduce_kernel<bf16, D, NR>>(2 * RCH * (int)sizeof(float));
+    e = reserve_lds<decode_reduce_kernel<bf16, D, NR, P>>(2 * RCH * (int)sizeof(float));
     if (e == hipSuccess)
-      hipLaunchKernelGGL((decode_reduce_kernel<bf16, D, NR>), dim3(rows), dim3(RTHREADS), stage, st, p);
+      hipLaunchKernelGGL((decode_reduce_kernel<bf16, D, NR, P>), dim3(rows), dim3(RTHREADS), stage, st, p);
   } else {
-    e = reserve_lds<decode_reduce_kernel<f16, D, NR>>(2 * RCH * (int)sizeof(float));
+    e = reserve_lds<decode_reduce_kernel<f16, D, NR, P>>(2 * RCH * (int)sizeof(float));
     if (e == hipSuccess)
-      hipLaunchKernelGGL((decode_reduce_kernel<f16, D, NR>), dim3(rows), dim3(RTHREADS), stage, st, p);
+      hipLaunchKernelGGL((decode_reduce_kernel<f16, D, NR, P>), dim3(rows), dim3(RTHREADS), stage, st, p);
   }
   CEA_REQUIRE(e == hipSuccess, CEA_ELAUNCH, "decode: cannot reserve %d bytes of LDS: %s",
               2 * RCH * (int)sizeof(float), hipGetErrorString(e));
   CEA_CHECK_LAUNCH("decode_reduce");
   return CEA_OK;
+}
+
+// One partition: the compact arguments (a launch copies its arguments, and every workgroup
+// starts by reading them): one token of 8 sequences of 4096 keys 13.3 -> 12.9 us, the one-token
+// decode block 23.4 -> 22.6 replayed.
+template <typename T, int D, int NR>
+int launch_nr(const DecodeParams& p, hipStream_t st) {
+  if (p.nparts > 1) return launch_parts<T, D, NR>(p, st);
+  DecodeParamsT<1> o;
+  o.nparts = 1;
+  o.q = p.q; o.q_pos = p.q_pos;
+  o.B = p.B; o.Sq = p.Sq; o.Hq = p.Hq; o.Hkv = p.Hkv; o.D = p.D;
+  o.qs_b = p.qs_b; o.qs_s = p.qs_s; o.qs_h = p.qs_h;
+  o.qps_b = p.qps_b; o.qps_s = p.qps_s;
+  o.k[0] = p.k[0]; o.v[0] = p.v[0]; o.k_pos[0] = p.k_pos[0];
+  o.Sk[0] = p.Sk[0];
+  o.part_out[0] = p.part_out[0]; o.part_lse[0] = p.part_lse[0];
+  for (int j = 0; j < 3; ++j) {
+    o.ks[0][j] = p.ks[0][j]; o.vs[0][j] = p.vs[0][j];
+    o.pos_[0][j] = p.pos_[0][j]; o.pls_[0][j] = p.pls_[0][j];
+  }
+  for (int j = 0; j < 2; ++j) {
+    o.kps[0][j] = p.kps[0][j];
+    o.chunk_begin[j] = p.chunk_begin[j];
+    o.item_begin[j] = p.item_begin[j];
+  }
+  o.chunk = p.chunk;
+  o.pair_rows = p.pair_rows;
+  o.scale = p.scale;
+  o.causal = p.causal;
+  o.in_dtype = p.in_dtype;
+  o.map = p.map;
+  o.partial = p.partial;
+  o.G = p.G; o.units = p.units; o.per_head = p.per_head;
+  o.out = p.out; o.lse = p.lse;
+  o.os_b = p.os_b; o.os_s = p.os_s; o.os_h = p.os_h;
+  o.ls_b = p.ls_b; o.ls_h = p.ls_h; o.ls_s = p.ls_s;
+  o.out_dtype = p.out_dtype;
+  o.accumulate = p.accumulate;
+  return launch_parts<T, D, NR>(o, st);
 }
 
 template <typename T, int D>

@@ -81,26 +81,29 @@ struct MergeParams {
 };
 
 // Split-KV decode over one or more KV partitions (short query blocks).
-struct DecodeParams {
+// MAXP: partitions the block has room for (kernels read it as an argument; the one-partition
+// form is a tenth of the size and its indices are constants).
+template <int MAXP> struct DecodeParamsT {
+  static constexpr int kParts = MAXP;
   int32_t nparts;
   const void* q;
   const int64_t* q_pos;
   int32_t B, Sq, Hq, Hkv, D;
   int64_t qs_b, qs_s, qs_h;
   int64_t qps_b, qps_s;
-  const void* k[CEA_MAX_PARTS];
-  const void* v[CEA_MAX_PARTS];
-  const int64_t* k_pos[CEA_MAX_PARTS];
-  int32_t Sk[CEA_MAX_PARTS];
-  int64_t ks[CEA_MAX_PARTS][3];
-  int64_t vs[CEA_MAX_PARTS][3];
-  int64_t kps[CEA_MAX_PARTS][2];
-  int32_t chunk_begin[CEA_MAX_PARTS + 1];  // prefix sum of key chunks per partition
+  const void* k[MAXP];
+  const void* v[MAXP];
+  const int64_t* k_pos[MAXP];
+  int32_t Sk[MAXP];
+  int64_t ks[MAXP][3];
+  int64_t vs[MAXP][3];
+  int64_t kps[MAXP][2];
+  int32_t chunk_begin[MAXP + 1];  // prefix sum of key chunks per partition
   int32_t chunk;                            // keys per chunk
   // set by the launcher: rows b < pair_rows take pairs of chunks as work items, item_begin is
   // the prefix sum of those pair items per partition
   int32_t pair_rows;
-  int32_t item_begin[CEA_MAX_PARTS + 1];
+  int32_t item_begin[MAXP + 1];
   double scale;
   int32_t causal;
   int32_t in_dtype;
@@ -115,10 +118,10 @@ struct DecodeParams {
   int32_t units;
   int32_t per_head;          // 1: units fastest in the grid (several units per KV head)
   // outputs of the reduction
-  void* part_out[CEA_MAX_PARTS];   // optional per-partition (out, lse), f32
-  void* part_lse[CEA_MAX_PARTS];
-  int64_t pos_[CEA_MAX_PARTS][3];  // per-partition out strides (b, s, h)
-  int64_t pls_[CEA_MAX_PARTS][3];  // per-partition lse strides (b, h, s)
+  void* part_out[MAXP];   // optional per-partition (out, lse), f32
+  void* part_lse[MAXP];
+  int64_t pos_[MAXP][3];  // per-partition out strides (b, s, h)
+  int64_t pls_[MAXP][3];  // per-partition lse strides (b, h, s)
   void* out;
   void* lse;
   int64_t os_b, os_s, os_h;
@@ -126,6 +129,7 @@ struct DecodeParams {
   int32_t out_dtype;
   int32_t accumulate;
 };
+using DecodeParams = DecodeParamsT<CEA_MAX_PARTS>;
 
 // Packing of one partial result into the all-gather message [B,Sq,H,D+1] (out | lse).
 struct PackParams {
