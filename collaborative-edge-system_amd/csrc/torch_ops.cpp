@@ -399,6 +399,14 @@ Tensor rmsnorm(const Tensor& x, const Tensor& weight_in, double eps) {
   return y;
 }
 
+// rmsnorm over the last dimension of x [..., C]: rows as a view (a copy only when the leading
+// dimensions do not collapse), the result in x's shape.
+Tensor rmsnorm_nd(const Tensor& x, const Tensor& weight, double eps) {
+  TORCH_CHECK_INDEX(x.dim() >= 1, "rmsnorm: x must have at least one dimension");
+  const Tensor rows = inner(x);
+  return rmsnorm(rows.reshape({-1, rows.size(-1)}), weight, eps).view(x.sizes());
+}
+
 std::vector<Tensor> rope_tables(const Tensor& pos_in, const Tensor& inv, at::ScalarType dtype) {
   const at::Device dev = device_of({&pos_in, &inv});
   const Tensor pos = as_i64(pos_in);
@@ -557,6 +565,7 @@ TORCH_LIBRARY(collab_edge, m) {
         "int kv_start, int kv_count) -> Tensor[]");
   m.def("ulysses_gather(Tensor[] outs, int start, int length) -> Tensor");
   m.def("rmsnorm(Tensor x, Tensor weight, float eps) -> Tensor");
+  m.def("rmsnorm_nd(Tensor x, Tensor weight, float eps) -> Tensor");
   m.def("rope_tables(Tensor positions, Tensor inv_freq, ScalarType dtype) -> Tensor[]");
   m.def("apply_rotary(Tensor x, Tensor cos, Tensor sin) -> Tensor");
   m.def("rmsnorm_rope(Tensor x, Tensor weight, float eps, Tensor positions, Tensor inv_freq, int num_heads) "
@@ -580,6 +589,7 @@ TORCH_LIBRARY_IMPL(collab_edge, CompositeExplicitAutograd, m) {
   m.impl("ulysses_scatter", ulysses_scatter);
   m.impl("ulysses_gather", ulysses_gather);
   m.impl("rmsnorm", rmsnorm);
+  m.impl("rmsnorm_nd", rmsnorm_nd);
   m.impl("rope_tables", rope_tables);
   m.impl("apply_rotary", apply_rotary);
   m.impl("rmsnorm_rope", rmsnorm_rope);

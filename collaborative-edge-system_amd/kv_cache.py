@@ -141,9 +141,9 @@ class LayerKVCache:
                 raise RuntimeError("nothing cached yet: pass like_k and like_pos to shape empty views")
             none_k = like_k.new_empty((like_k.shape[0], 0, *like_k.shape[2:]))
             return none_k, none_k, like_pos.new_empty((like_pos.shape[0], 0))
-        n = self.length
-        return (self._k[:, :, :n].transpose(1, 2), self._v[:, :, :n].transpose(1, 2),
-                self._pos[:, :n])
+        n = min(self.length, self._k.size(2))
+        return (self._k.narrow(2, 0, n).transpose(1, 2), self._v.narrow(2, 0, n).transpose(1, 2),
+                self._pos.narrow(1, 0, n))
 
     def nbytes(self) -> int:
         """Bytes of the cached tokens' keys and values (not the unused slots)."""

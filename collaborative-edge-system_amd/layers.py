@@ -64,7 +64,7 @@ def _rows(x: torch.Tensor) -> torch.Tensor:
 
 def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
     """Functional RMSNorm with the reference's rounding (llama.py:58-61)."""
-    return nat.ops().rmsnorm(_rows(x), weight, float(eps)).view(x.shape)
+    return nat.ops().rmsnorm_nd(x, weight, float(eps))
 
 
 class RMSNorm(nn.Module):

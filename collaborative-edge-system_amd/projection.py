@@ -33,7 +33,7 @@ from .layers import ACTIVATION_CODES
 
 
 def _check_operands(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], what: str):
-    if weight.dim() != 2 or x.dim() < 1 or x.shape[-1] != weight.shape[1]:
+    if weight.dim() != 2 or x.dim() < 1 or x.size(-1) != weight.size(1):
         raise ValueError(f"{what}: x [..., {x.shape[-1] if x.dim() else '?'}] does not match "
                          f"weight {tuple(weight.shape)}")
     if weight.dtype != x.dtype or (bias is not None and bias.dtype != x.dtype):
@@ -47,7 +47,8 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] =
     """``F.linear(x, weight, bias)`` for ``x [..., K]``, ``weight [N, K]``, ``bias [N]`` on the
     device; ``out`` may be a preallocated ``[M, N]`` buffer (M = product of x's leading sizes,
     any row stride)."""
-    nat.require_device(x, weight, bias, out)
+    if not (x.is_cuda and weight.is_cuda and out is None and (bias is None or bias.is_cuda)):
+        nat.require_device(x, weight, bias, out)  # (the operator checks that the devices agree)
     _check_operands(x, weight, bias, "linear")
     if out is None:
         return nat.ops().linear(x, weight, bias)
@@ -61,7 +62,7 @@ def fused_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Ten
     (tensor_parallel.py:294-295)."""
     if sum(split_sizes) != weight.shape[0]:
         raise ValueError(f"split sizes {list(split_sizes)} do not add up to {weight.shape[0]}")
-    return list(linear(x, weight, bias).split(list(split_sizes), dim=-1))
+    return list(torch.split_with_sizes(linear(x, weight, bias), list(split_sizes), -1))
 
 
 def linear_gated(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor,
