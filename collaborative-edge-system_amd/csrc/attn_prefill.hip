@@ -152,12 +152,14 @@ __global__ __launch_bounds__(NTHREADS, 2) void attn_prefill_kernel(const AttnPar
   const int g = lane >> 5;   // half of the wave
 
   // ---- XCD-aware work mapping (blocks are dispatched round-robin over 8 XCDs): the query
-  // heads of one KV head stay on one XCD, whose L2 then serves their K and V, and each XCD
-  // starts its heaviest (latest causal) query blocks first, all heads' before any lighter one,
-  // so the blocks left for the end are the short ones.  The KV heads are dealt to the XCDs in
-  // turn, so a batch row shorter than the others leaves work on every XCD.  With the heads in
-  // turn instead (a head's blocks, then the next head's), two prompts of 2000 tokens (32/8
-  // heads) took 130 us, now 79, and 30000 of one rank of 4 (14/2 heads) 1272, now 723.
+  // heads of one KV head stay on one XCD, whose L2 then serves their K and V.  The KV heads are
+  // dealt to the XCDs in turn, so a batch row shorter than the others leaves work on every XCD.
+  // An XCD takes as many query heads together as their KV heads fit its L2 (order_units) and
+  // starts the heaviest (latest causal) query blocks of all of them before any lighter one, so
+  // the blocks left for the end are the short ones.  Measured (us): two prompts of 2000 tokens
+  // (32/8 heads) one head after the other 118, all together 87; two of 6000, whose KV heads of
+  // 3 MB do not fit together, 457 one head after the other, 514 all together, 430 by KV head (in
+  // the order of the grid, 594); 30000 tokens of one rank of 4 (14/2 heads) 1272 -> 723.
   // A key-split launch repeats the grid once per split, split slowest, so the workgroups of
   // one split and KV head (which read the same tiles) stay together as well.  A workgroup
   // holds hp query heads of one KV head's group (NWAVES / hp waves and BM / hp rows each), so
@@ -182,16 +184,18 @@ __global__ __launch_bounds__(NTHREADS, 2) void attn_prefill_kernel(const AttnPar
     b = bh / ngroups;
   } else {
     int unit;
-    const int kv_heads = p.B * p.Hkv;
-    if (p.map.group > 0 && (kv_heads & 7) == 0) {
-      const int per_xcd = units >> 3, per_kv = ngroups / p.Hkv;
-      const int i = blk >> 3, u = i % per_xcd;
-      qb = i / per_xcd;
-      unit = ((blk & 7) + 8 * (u / per_kv)) * per_kv + u % per_kv;
-    } else if ((units & 7) == 0) {
+    if ((units & 7) == 0) {
       const int per_xcd = units >> 3, i = blk >> 3;
-      qb = i / per_xcd;
-      unit = (blk & 7) * per_xcd + i % per_xcd;
+      const int set = i / (p.order_units * nqb);   // query heads taken together
+      const int r = i - set * p.order_units * nqb;
+      const int size = min(p.order_units, per_xcd - set * p.order_units);
+      const int u = set * p.order_units + r % size;
+      qb = r / size;
+      const int per_kv = p.map.group > 0 ? ngroups / p.Hkv : 1;
+      if (p.map.group > 0 && ((p.B * p.Hkv) & 7) == 0)
+        unit = ((blk & 7) + 8 * (u / per_kv)) * per_kv + u % per_kv;
+      else
+        unit = (blk & 7) * per_xcd + u;
     } else {
       qb = blk / units;
       unit = blk % units;
@@ -200,6 +204,9 @@ __global__ __launch_bounds__(NTHREADS, 2) void attn_prefill_kernel(const AttnPar
     hg = unit % ngroups;
     b = unit / ngroups;
   }
+  // (in scalar registers: left to itself the compiler kept the merged paths' values in vector
+  // registers and the tile loop lost 2 %)
+  qb = uniform(qb), b = uniform(b), hg = uniform(hg), split = uniform(split);
   const int waves_ph = NWAVES / hp;
   const int h = hg * hp + wave / waves_ph;   // this wave's query head
   const int kvh = p.map.kv_of(hg * hp);      // one KV head for the whole workgroup
@@ -608,8 +615,22 @@ __global__ __launch_bounds__(NTHREADS, 2) void attn_prefill_kernel(const AttnPar
 }
 
 template <typename T, int D, bool MULTI>
-int launch_typed(const AttnParams& p, const KvSegs& segs, hipStream_t st) {
+int launch_typed(const AttnParams& params, const KvSegs& segs, hipStream_t st) {
+  AttnParams p = params;
   const int hp = MULTI ? 1 : std::max(p.heads_per_wg, 1);
+  // query-head units an XCD takes together: whole KV heads, as many as 5 MB hold (a 4 MB L2 does
+  // not mind a little more: three heads of 1.5 MB 171 us together, 237 as two and one; two of
+  // 3 MB 514 together, 430 one by one), in sets of even size
+  const int64_t kv_bytes = std::max<int64_t>((int64_t)p.ntiles * BN * Layout<D>::KROW * 2, 1);
+  const int64_t per_kv = p.map.group > 0 ? p.Hq / hp / p.Hkv : 1;
+  const int64_t heads = std::max<int64_t>(((int64_t)p.B * (p.Hq / hp) + 8 * per_kv - 1) / (8 * per_kv), 1);
+  const int64_t fit = std::max<int64_t>(((int64_t)5 << 20) / kv_bytes, 1);
+  const int64_t sets = (heads + fit - 1) / fit;
+  p.order_units = (int)((heads + sets - 1) / sets * per_kv);
+  // one sequence, one block: an XCD holds one KV head or part of one, and its query heads one
+  // after the other measured 1 % faster (6000 tokens, 32/8 heads 313 against 317; the ring
+  // share's blocks 1 % slower)
+  if (!MULTI && p.B == 1 && heads == 1) p.order_units = 1;
   const int nqb = (p.Sq + BM / hp - 1) / (BM / hp);
   const int64_t total = (int64_t)nqb * (p.Hq / hp) * p.B * (MULTI ? 1 : std::max(p.splits, 1));
   if (total == 0) return CEA_OK;

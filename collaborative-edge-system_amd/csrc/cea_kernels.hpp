@@ -43,6 +43,9 @@ struct AttnParams {
   // prefill workgroups hold this many query heads of one KV head's group (0 or 1: one), each
   // with 1 / heads_per_wg of the workgroup's query rows
   int32_t heads_per_wg;
+  // set by the prefill launcher: workgroup columns (query heads / heads_per_wg) an XCD works
+  // through together
+  int32_t order_units;
 };
 
 // KV blocks of one prefill launch, in the order their tiles are visited (a ring share's
