@@ -130,9 +130,11 @@ template <int LPT> __device__ __forceinline__ void wait_tiles_ahead(int ahead) {
   else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
+// FINE: the probabilities enter the value product as the sum of two 16-bit numbers, p and what
+// rounding it left (22 bits of f16, 16 of bf16), in a second pass over V.
 // MULTI: the launch streams several KV blocks (segs.n > 1); otherwise block 0 only, whose
 // addresses the compiler keeps in registers for the whole kernel.
-template <typename T, int D, bool MULTI>
+template <typename T, int D, bool MULTI, bool FINE>
 __global__ __launch_bounds__(NTHREADS, 2) void attn_prefill_kernel(const AttnParams p,
                                                                    const KvSegs segs) {
   typedef Layout<D> L;
@@ -425,12 +427,23 @@ __global__ __launch_bounds__(NTHREADS, 2) void attn_prefill_kernel(const AttnPar
         pr[kb * 16 + e] = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[kb][e], c, -m_use));
         pf[kb * 2 + (e >> 3)][e & 7] = (T)pr[kb * 16 + e];
       }
-    // f32 row sum as a tree of independent adds
+    // f32 row sum as a tree of independent adds (FINE still needs the probabilities)
+    if constexpr (FINE) {
+      float rs[16];
 #pragma unroll
-    for (int w = 16; w >= 1; w >>= 1)
+      for (int e = 0; e < 16; ++e) rs[e] = pr[e] + pr[e + 16];
 #pragma unroll
-      for (int e = 0; e < w; ++e) pr[e] += pr[e + w];
-    l_run += pr[0];
+      for (int w = 8; w >= 1; w >>= 1)
+#pragma unroll
+        for (int e = 0; e < w; ++e) rs[e] += rs[e + w];
+      l_run += rs[0];
+    } else {
+#pragma unroll
+      for (int w = 16; w >= 1; w >>= 1)
+#pragma unroll
+        for (int e = 0; e < w; ++e) pr[e] += pr[e + w];
+      l_run += pr[0];
+    }
     // O^T += V^T . P^T: fragment of step s holds keys s*16 + {g*4..+3, 8+g*4..+3}
 #pragma unroll
     for (int dt = 0; dt < D / 32; ++dt) {
@@ -453,6 +466,18 @@ __global__ __launch_bounds__(NTHREADS, 2) void attn_prefill_kernel(const AttnPar
       }
     }
     __builtin_amdgcn_sched_group_barrier(0x008, 4, 1);
+    if constexpr (FINE) {
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int e = 0; e < 32; ++e) pf[e >> 3][e & 7] = (T)(pr[e] - to_f32<T>(pf[e >> 3][e & 7]));
+#pragma unroll
+      for (int dt = 0; dt < D / 32; ++dt)
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+          oacc[dt] = Mfma<T>::run(read_tr_frag<frag>(sb + s * 16 * L::KROW + v_raddr[dt],
+                                                     sb + (s * 16 + 8) * L::KROW + v_raddr[dt]),
+                                  pf[s], oacc[dt]);
+    }
   };
 
   // ---- passes over the key block: list the tiles this workgroup needs, then stream them.
@@ -614,7 +639,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void attn_prefill_kernel(const AttnPar
   }
 }
 
-template <typename T, int D, bool MULTI>
+template <typename T, int D, bool MULTI, bool FINE>
 int launch_typed(const AttnParams& params, const KvSegs& segs, hipStream_t st) {
   AttnParams p = params;
   const int hp = MULTI ? 1 : std::max(p.heads_per_wg, 1);
@@ -635,10 +660,10 @@ int launch_typed(const AttnParams& params, const KvSegs& segs, hipStream_t st) {
   const int64_t total = (int64_t)nqb * (p.Hq / hp) * p.B * (MULTI ? 1 : std::max(p.splits, 1));
   if (total == 0) return CEA_OK;
   CEA_REQUIRE(total < (int64_t)1 << 31, CEA_EUNSUPPORTED, "attention: grid too large");
-  const hipError_t e = reserve_lds<attn_prefill_kernel<T, D, MULTI>>(Layout<D>::LDS_BYTES);
+  const hipError_t e = reserve_lds<attn_prefill_kernel<T, D, MULTI, FINE>>(Layout<D>::LDS_BYTES);
   CEA_REQUIRE(e == hipSuccess, CEA_ELAUNCH, "attention: cannot reserve %d bytes of LDS: %s",
               Layout<D>::LDS_BYTES, hipGetErrorString(e));
-  hipLaunchKernelGGL((attn_prefill_kernel<T, D, MULTI>), dim3((unsigned)total), dim3(NTHREADS),
+  hipLaunchKernelGGL((attn_prefill_kernel<T, D, MULTI, FINE>), dim3((unsigned)total), dim3(NTHREADS),
                      Layout<D>::LDS_BYTES, st, p, segs);
   CEA_CHECK_LAUNCH("attention_prefill");
   return CEA_OK;
@@ -702,7 +727,7 @@ static bool prefill_block_ok(const AttnParams& p, const KvSeg& g) {
   // key positions are fetched two (16 bytes) per lane, which needs no more than their own
   // alignment: contiguous along the keys, any batch stride and first key.  (Asking for 16-byte
   // aligned rows sent every block with an odd number of keys to the generic kernel: one of
-  // eight ranks' share of 3000 tokens took 40 ms there, 114 us here.)
+  // eight ranks' share of 3000 tokens took 40 ms there, 148 us here.)
   if (g.kps_s != 1) return false;
   // tiles are addressed from 64-bit bases with 32-bit offsets inside one tile, so a block may
   // span any number of bytes; list entries hold a tile of the block in 24 bits
@@ -753,18 +778,31 @@ bool prefill_segs_supported(const AttnParams& p, const KvSegs& segs) {
   return tiles == p.ntiles && tiles < ((int64_t)1 << 24);
 }
 
-template <bool MULTI>
-static int launch_dispatch(const AttnParams& p, const KvSegs& segs, hipStream_t st) {
+template <bool MULTI, bool FINE>
+static int launch_as(const AttnParams& p, const KvSegs& segs, hipStream_t st) {
   if (p.in_dtype == CEA_BF16) {
-    if (p.D == 128) return launch_typed<bf16, 128, MULTI>(p, segs, st);
-    if (p.D == 64) return launch_typed<bf16, 64, MULTI>(p, segs, st);
+    if (p.D == 128) return launch_typed<bf16, 128, MULTI, FINE>(p, segs, st);
+    if (p.D == 64) return launch_typed<bf16, 64, MULTI, FINE>(p, segs, st);
   } else if (p.in_dtype == CEA_F16) {
-    if (p.D == 128) return launch_typed<f16, 128, MULTI>(p, segs, st);
-    if (p.D == 64) return launch_typed<f16, 64, MULTI>(p, segs, st);
+    if (p.D == 128) return launch_typed<f16, 128, MULTI, FINE>(p, segs, st);
+    if (p.D == 64) return launch_typed<f16, 64, MULTI, FINE>(p, segs, st);
   }
   set_error("attention: MFMA path does not cover dtype %s, head size %d",
             dtype_name(p.in_dtype), p.D);
   return CEA_EUNSUPPORTED;
+}
+
+// Blocks whose position rows are not 16-byte aligned (an odd number of keys, an odd first slot)
+// used to run on the generic kernel, which keeps its probabilities in f32: they take the FINE
+// form, so their results are no further from exact than they were (f16, 701 tokens, 32/8 heads,
+// 2-norm: 2.00e-4 there and here, 2.9e-4 without the second pass; 9393 us there, 47 here, 34
+// without).
+template <bool MULTI>
+static int launch_dispatch(const AttnParams& p, const KvSegs& segs, hipStream_t st) {
+  bool fine = false;
+  for (int i = 0; i < segs.n; ++i)
+    fine = fine || segs.seg[i].kps_b % 2 || !al16(segs.seg[i].k_pos);
+  return fine ? launch_as<MULTI, true>(p, segs, st) : launch_as<MULTI, false>(p, segs, st);
 }
 
 int launch_attn_prefill_mfma(const AttnParams& p, hipStream_t st) {
