@@ -138,3 +138,31 @@ def test_key_split_and_subgroup_decode_replays(cea, dev):
 
     bq, bk, bv, bpos = _attn_inputs(dev, 2048, 9)
     _replays_match(step, lambda: cea.attention_with_lse(bq, bk, bv, bpos, bpos))
+
+
+@pytest.mark.parametrize("tokens", [20, 300])
+def test_graph_of_projections(cea, dev, tokens):
+    """The few-token kernel and a K-split launch (its sums in the stream's workspace) captured
+    together: replays on changed inputs, with eager calls of another size between them, equal
+    the eager results."""
+    g = torch.Generator().manual_seed(tokens)
+    x = torch.randn(tokens, 2048, generator=g).to(torch.bfloat16).to(dev)
+    w = (torch.randn(512, 2048, generator=g) / 45).to(torch.bfloat16).to(dev)
+    wd = (torch.randn(2048, 256, generator=g) / 16).to(torch.bfloat16).to(dev)
+    step = lambda t: cea.linear(cea.linear_gated(t, w[:256], w[256:]), wd)
+    stream = torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(stream):
+        step(x)
+        stream.synchronize()
+        with torch.cuda.graph(graph, stream=stream):
+            y = step(x)
+    for i in range(3):
+        x.copy_(torch.randn(tokens, 2048, generator=g).to(torch.bfloat16))
+        want = step(x).clone()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want), i
+        step(torch.randn(900, 2048, device=dev).to(torch.bfloat16))
+        torch.cuda.synchronize()
