@@ -230,6 +230,7 @@ template <int MODE, int ACT>
 int launch_f32(const GemmParams& p, hipStream_t st) {
   int rb = 4, tb = 4;
   blocks_f32<MODE>(p, rb, tb);
+  if (ceil_div(p.M, tb * 16) > 65535) tb = 4;   // the second grid dimension
   CEA_REQUIRE(ceil_div(p.M, tb * 16) <= 65535, CEA_EUNSUPPORTED, "linear: %d rows exceed the f32 kernel's grid",
               p.M);
   if constexpr (MODE == kPlain)
