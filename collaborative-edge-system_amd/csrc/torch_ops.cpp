@@ -8,13 +8,12 @@
 // CEA_EINVAL -> ValueError, CEA_EUNSUPPORTED -> NotImplementedError, others -> RuntimeError.
 // Host (CPU) tensors are refused with RuntimeError: there is no host path.
 #include <ATen/ATen.h>
+#include <c10/core/Allocator.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/library.h>
 
 #include <algorithm>
-#include <map>
-#include <mutex>
 #include <string>
 #include <utility>
 #include <vector>
@@ -94,36 +93,25 @@ void* stream_of(const at::Device& d) {
   return (void*)c10::hip::getCurrentHIPStream(d.index()).stream();
 }
 
-// The kernels' workspace: one buffer per (device, stream), grown to the largest request seen
-// and then reused by every call on that stream (calls on one stream run in order, so a call
-// never overwrites scratch a queued call still reads).  A grown-out buffer returns to
-// PyTorch's caching allocator, which hands its memory out again only in stream order - unless
-// a HIP graph capture may have recorded it: graph replays keep writing to the captured
-// address whatever the allocator has since handed it to, so such a buffer is kept alive
-// (retired, never freed) when a larger one replaces it.
-struct WsEntry {
-  Tensor t;
-  bool captured = false;  // used while its stream was capturing a graph
+// The scratch of one call, on the current stream.  Each call takes its own from PyTorch's caching
+// allocator, which hands freed memory out again in stream order only and serves a capture from
+// the graph's own pool.  Scratch kept per stream would be shared: a call of several launches
+// (tile summaries or partial sums, then the kernel that reads them) does not hold its stream, so
+// another thread's call on it may come in between, and graphs captured on one stream may be
+// replayed on several.
+struct Scratch {
+  c10::DataPtr mem;
+  size_t size = 0;
+  void* data() const { return mem.get(); }
 };
-std::mutex g_ws_mu;
-std::map<std::pair<int, void*>, WsEntry> g_ws;
-std::vector<Tensor> g_ws_retired;
 
-Tensor workspace(size_t bytes, const at::Device& d) {
-  void* st = stream_of(d);
-  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  const bool capturing =
-      hipStreamIsCapturing((hipStream_t)st, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone;
-  const int64_t want = (int64_t)std::max<size_t>((bytes + 4095) & ~(size_t)4095, 4096);
-  std::lock_guard<std::mutex> lock(g_ws_mu);
-  WsEntry& e = g_ws[{(int)d.index(), st}];
-  if (!e.t.defined() || e.t.numel() < want) {
-    if (e.t.defined() && (e.captured || capturing)) g_ws_retired.push_back(e.t);
-    e.t = at::empty({want}, at::TensorOptions().dtype(at::kByte).device(d));
-    e.captured = false;
-  }
-  e.captured = e.captured || capturing;
-  return e.t;
+// (the device is the current one: every operator holds a DeviceGuard when it asks)
+Scratch workspace(size_t bytes) {
+  static c10::Allocator* const device_memory = c10::GetAllocator(c10::DeviceType::CUDA);
+  Scratch s;
+  s.size = std::max<size_t>((bytes + 4095) & ~(size_t)4095, 4096);
+  s.mem = device_memory->allocate(s.size);
+  return s;
 }
 
 // q / k / v style operands need a unit innermost stride
@@ -159,12 +147,12 @@ std::vector<Tensor> attention(const Tensor& q_in, const Tensor& k_in, const Tens
   Tensor lse = with_lse ? at::empty({B, Hq, Sq}, o_opts.dtype(acc)) : Tensor();
   c10::DeviceGuard guard(dev);
   const std::vector<int32_t> m = map_of(kv_map);
-  Tensor ws = workspace(cea_attention_workspace_bytes(B, Sq, Hq, Sk, Hkv, D, code_of(q.scalar_type())), dev);
+  const Scratch ws = workspace(cea_attention_workspace_bytes(B, Sq, Hq, Sk, Hkv, D, code_of(q.scalar_type())));
   cea_tensor a[5] = {arg(q), arg(k), arg(v), arg(qp), arg(kp)};
   cea_tensor o = arg(out), l = with_lse ? arg(lse) : cea_tensor{};
   check_rc(cea_attention_with_lse(&a[0], &a[1], &a[2], &a[3], &a[4], causal ? 1 : 0, scale,
                                   m.empty() ? nullptr : m.data(), (int32_t)m.size(), &o,
-                                  with_lse ? &l : nullptr, 0, ws.data_ptr(), (size_t)ws.numel(),
+                                  with_lse ? &l : nullptr, 0, ws.data(), ws.size,
                                   stream_of(dev)),
            "attention_with_lse");
   if (with_lse) return {out, lse};
@@ -182,22 +170,21 @@ void attention_into(Tensor out, Tensor lse, const Tensor& q_in, const Tensor& k_
   TORCH_CHECK_VALUE(q.dim() == 4 && k.dim() == 4, "q and k must be [B, S, H, D]");
   c10::DeviceGuard guard(dev);
   const std::vector<int32_t> m = map_of(kv_map);
-  Tensor ws = workspace(cea_attention_workspace_bytes(q.size(0), q.size(1), q.size(2), k.size(1), k.size(2),
-                                                      q.size(3), code_of(q.scalar_type())),
-                        dev);
+  const Scratch ws = workspace(cea_attention_workspace_bytes(q.size(0), q.size(1), q.size(2), k.size(1),
+                                                             k.size(2), q.size(3), code_of(q.scalar_type())));
   cea_tensor a[5] = {arg(q), arg(k), arg(v), arg(qp), arg(kp)};
   cea_tensor o = arg(out), l = arg(lse);
   if (fin.defined()) {
     cea_tensor f = arg(fin);
     check_rc(cea_attention_merge_final(&a[0], &a[1], &a[2], &a[3], &a[4], causal ? 1 : 0, scale,
                                        m.empty() ? nullptr : m.data(), (int32_t)m.size(), &o, &l, &f,
-                                       ws.data_ptr(), (size_t)ws.numel(), stream_of(dev)),
+                                       ws.data(), ws.size, stream_of(dev)),
              "attention_merge_final");
     return;
   }
   check_rc(cea_attention_with_lse(&a[0], &a[1], &a[2], &a[3], &a[4], causal ? 1 : 0, scale,
                                   m.empty() ? nullptr : m.data(), (int32_t)m.size(), &o, &l,
-                                  accumulate ? 1 : 0, ws.data_ptr(), (size_t)ws.numel(), stream_of(dev)),
+                                  accumulate ? 1 : 0, ws.data(), ws.size, stream_of(dev)),
            "attention_with_lse");
 }
 
@@ -256,7 +243,7 @@ std::vector<Tensor> partitioned(const Tensor& q_in, const Tensor& q_pos_in, at::
   for (const Tensor& k : ks) sks.push_back(k.size(1));
   const size_t ws_bytes = cea_partitioned_attention_workspace_bytes(
       (int32_t)n, sks.data(), B, Sq, Hq, ks[0].size(2), D, code_of(q.scalar_type()));
-  Tensor ws = workspace(ws_bytes, dev);
+  const Scratch ws = workspace(ws_bytes);
   const std::vector<int32_t> m = map_of(kv_map);
   cea_tensor qa = arg(q), qpa = arg(qp), o = arg(out);
   cea_tensor l = with_lse ? arg(lse) : cea_tensor{};
@@ -265,7 +252,7 @@ std::vector<Tensor> partitioned(const Tensor& q_in, const Tensor& q_pos_in, at::
   check_rc(cea_partitioned_attention(&qa, (int32_t)n, ka.data(), va.data(), &qpa, pa.data(), causal ? 1 : 0,
                                      scale, m.empty() ? nullptr : m.data(), (int32_t)m.size(),
                                      with_parts ? poa.data() : nullptr, with_parts ? pla.data() : nullptr, &o,
-                                     with_lse ? &l : nullptr, ws.data_ptr(), (size_t)ws.numel(), stream_of(dev)),
+                                     with_lse ? &l : nullptr, ws.data(), ws.size, stream_of(dev)),
            "partitioned_attention");
   std::vector<Tensor> res{out};
   if (with_lse) res.push_back(lse);
@@ -307,10 +294,10 @@ std::vector<Tensor> ring(const Tensor& q_in, const Tensor& q_pos_in, at::TensorL
   const size_t ws_bytes = cea_ring_attention_workspace_bytes(
       &qa, (int32_t)n, ka.data(), va.data(), &qpa, pa.data(), causal ? 1 : 0,
       m.empty() ? nullptr : m.data(), (int32_t)m.size(), &o, with_lse ? &l : nullptr);
-  Tensor ws = workspace(ws_bytes, dev);
+  const Scratch ws = workspace(ws_bytes);
   check_rc(cea_ring_attention(&qa, (int32_t)n, ka.data(), va.data(), &qpa, pa.data(), causal ? 1 : 0, scale,
                               m.empty() ? nullptr : m.data(), (int32_t)m.size(), &o,
-                              with_lse ? &l : nullptr, ws.data_ptr(), (size_t)ws.numel(), stream_of(dev)),
+                              with_lse ? &l : nullptr, ws.data(), ws.size, stream_of(dev)),
            "ring_attention");
   if (with_lse) return {out, lse};
   return {out};
@@ -464,11 +451,11 @@ std::vector<int64_t> out_shape(const Tensor& x, int64_t n) {
   return s;
 }
 
-// The scratch of a projection to n columns (undefined when it needs none).
-Tensor linear_workspace(const Tensor& x2, int64_t n, int gated, const at::Device& dev) {
+// The scratch of a projection to n columns (null when it needs none).
+Scratch linear_workspace(const Tensor& x2, int64_t n, int gated) {
   const size_t bytes =
       cea_linear_workspace_bytes(x2.size(0), n, x2.size(1), code_of(x2.scalar_type()), gated);
-  return bytes ? workspace(bytes, dev) : Tensor();
+  return bytes ? workspace(bytes) : Scratch();
 }
 
 void linear_call(const Tensor& x2, const Tensor& weight, const c10::optional<Tensor>& bias,
@@ -476,11 +463,10 @@ void linear_call(const Tensor& x2, const Tensor& weight, const c10::optional<Ten
   const Tensor w = inner(weight);
   const Tensor b = bias ? inner(*bias) : Tensor();
   c10::DeviceGuard guard(dev);
-  const Tensor ws = linear_workspace(x2, w.size(0), 0, dev);
+  const Scratch ws = linear_workspace(x2, w.size(0), 0);
   cea_tensor a = arg(x2), c = arg(w), d, e = arg(y2);
   if (b.defined()) d = arg(b);
-  check_rc(cea_linear_ws(&a, &c, b.defined() ? &d : nullptr, &e, ws.defined() ? ws.data_ptr() : nullptr,
-                         ws.defined() ? (size_t)ws.numel() : 0, stream_of(dev)),
+  check_rc(cea_linear_ws(&a, &c, b.defined() ? &d : nullptr, &e, ws.data(), ws.size, stream_of(dev)),
            "linear");
 }
 
@@ -521,10 +507,10 @@ Tensor linear_gated(const Tensor& x, const Tensor& w_gate, const Tensor& w_up,
   cea_tensor f, g;
   if (bg.defined()) f = arg(bg);
   if (bu.defined()) g = arg(bu);
-  const Tensor ws = linear_workspace(x2, w_gate.size(0), 1, dev);
+  const Scratch ws = linear_workspace(x2, w_gate.size(0), 1);
   check_rc(cea_linear_gated_ws(&a, &c, &d, bg.defined() ? &f : nullptr, bu.defined() ? &g : nullptr, &e,
-                               (int32_t)act, ws.defined() ? ws.data_ptr() : nullptr,
-                               ws.defined() ? (size_t)ws.numel() : 0, stream_of(dev)),
+                               (int32_t)act, ws.data(), ws.size,
+                               stream_of(dev)),
            "linear_gated");
   return y;
 }

@@ -4,10 +4,12 @@
   equal the eager results on every replay, with eager work on the device between the
   replays (the kernels write every scratch value they read in the same call and record no
   memset).
-* The operator library's per-stream workspace: a buffer that a capture recorded stays
-  allocated when a later, larger call on that stream replaces it, so replays never write into
-  memory the allocator has handed out again.
+* The operators' scratch: what a capture recorded belongs to its graph, so replays never write
+  into memory the allocator has handed out again, graphs captured on one stream can be replayed
+  on two, and calls of two threads on one stream do not share it.
 """
+
+import threading
 
 import pytest
 import torch
@@ -27,15 +29,15 @@ def _attn_inputs(dev, s, seed, hq=4, hkv=2, d=128):
 def test_captured_workspace_survives_growth(cea, dev):
     s = torch.cuda.Stream(dev)
     q, k, v, pos = _attn_inputs(dev, 256, 1)
-    bq, bk, bv, bpos = _attn_inputs(dev, 16384, 2)  # 256 tiles: a larger workspace
+    bq, bk, bv, bpos = _attn_inputs(dev, 16384, 2)  # 256 tiles: more scratch
     with torch.cuda.stream(s):
-        ref_o, ref_l = cea.attention_with_lse(q, k, v, pos, pos)  # the stream's first workspace
+        ref_o, ref_l = cea.attention_with_lse(q, k, v, pos, pos)
     s.synchronize()
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph, stream=s):
         out, lse = cea.attention_with_lse(q, k, v, pos, pos)
     with torch.cuda.stream(s):
-        cea.attention_with_lse(bq, bk, bv, bpos, bpos)  # replaces the captured workspace
+        cea.attention_with_lse(bq, bk, bv, bpos, bpos)
         fillers = [torch.full((4096,), 7, dtype=torch.uint8, device=dev) for _ in range(32)]
     s.synchronize()
     for i in range(3):
@@ -142,7 +144,7 @@ def test_key_split_and_subgroup_decode_replays(cea, dev):
 
 @pytest.mark.parametrize("tokens", [20, 300])
 def test_graph_of_projections(cea, dev, tokens):
-    """The few-token kernel and a K-split launch (its sums in the stream's workspace) captured
+    """The few-token kernel and a K-split launch (its sums in the graph's memory) captured
     together: replays on changed inputs, with eager calls of another size between them, equal
     the eager results."""
     g = torch.Generator().manual_seed(tokens)
@@ -166,3 +168,80 @@ def test_graph_of_projections(cea, dev, tokens):
         assert torch.equal(y, want), i
         step(torch.randn(900, 2048, device=dev).to(torch.bfloat16))
         torch.cuda.synchronize()
+
+
+# calls of several launches that pass scratch from one to the next: a K-split projection (plain and
+# gated), key-split prefill, one-launch prefill and split-KV decode
+def _scratch_calls(cea, dev, seed):
+    g = torch.Generator().manual_seed(seed)
+    rand = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16).to(dev)
+    x, w, wd = rand(300, 2048), rand(1024, 2048) / 45, rand(512, 4096) / 64
+    xd = rand(300, 4096)
+    q, k, v, pos = _attn_inputs(dev, 3000, seed + 1, hq=8, hkv=2)
+    return [
+        lambda: cea.linear(xd, wd),
+        lambda: cea.linear_gated(x, w[:512], w[512:]),
+        lambda: cea.attention.attention(q[:, -96:], k, v, pos[:, -96:], pos),
+        lambda: cea.attention.attention(q[:, :700], k[:, :700], v[:, :700], pos[:, :700], pos[:, :700]),
+        lambda: cea.attention.attention(q[:, -1:], k, v, pos[:, -1:], pos),
+    ]
+
+
+def test_two_threads_on_one_stream(cea, dev):
+    """Each thread gets its own results, whatever call of the other thread is enqueued between
+    the launches of one of its calls."""
+    calls = [_scratch_calls(cea, dev, 10), _scratch_calls(cea, dev, 20)]
+    want = [[f() for f in c] for c in calls]
+    torch.cuda.synchronize()
+    wrong, start = [], threading.Barrier(2)
+
+    def work(t):
+        with torch.cuda.stream(stream):
+            start.wait(timeout=30)
+            for i in range(40):
+                for j in range(len(calls[t])):
+                    f = calls[t][(j + t) % len(calls[t])]
+                    got.append((t, (j + t) % len(calls[t]), f()))
+
+    stream = torch.cuda.Stream(dev)
+    got = []
+    threads = [threading.Thread(target=work, args=(t,)) for t in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(timeout=60)
+        assert not t.is_alive()
+    torch.cuda.synchronize()
+    assert len(got) == 2 * 40 * 5
+    wrong = [(t, j) for t, j, y in got if not torch.equal(y, want[t][j])]
+    assert not wrong, wrong[:10]
+
+
+def test_graphs_of_one_stream_replayed_on_two(cea, dev):
+    """Two graphs captured on the same stream own their scratch: replayed at the same time on two
+    streams, with eager calls on the capture stream, each gives its own results."""
+    calls = [_scratch_calls(cea, dev, 30), _scratch_calls(cea, dev, 40)]
+    want = [[f() for f in c] for c in calls]
+    torch.cuda.synchronize()
+    capture = torch.cuda.Stream(dev)
+    graphs, outs = [], []
+    for c in calls:
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=capture):
+            outs.append([f() for f in c])
+        graphs.append(graph)
+    streams = [torch.cuda.Stream(dev) for _ in graphs]
+    for i in range(10):
+        for ys in outs:
+            for y in ys:
+                y.zero_()
+        torch.cuda.synchronize()
+        for graph, s in zip(graphs, streams):
+            with torch.cuda.stream(s):
+                graph.replay()
+        with torch.cuda.stream(capture):
+            eager = [f() for f in calls[0]]
+        torch.cuda.synchronize()
+        for ys, ws in zip(outs + [eager], want + [want[0]]):
+            for j, (y, w) in enumerate(zip(ys, ws)):
+                assert torch.equal(y, w), (i, j)
