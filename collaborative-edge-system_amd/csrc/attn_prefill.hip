@@ -35,6 +35,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "cea_kernels.hpp"
 #include "cea_lds_dma.hpp"
@@ -130,11 +131,17 @@ template <int LPT> __device__ __forceinline__ void wait_tiles_ahead(int ahead) {
   else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
-// FINE: the probabilities enter the value product as the sum of two 16-bit numbers, p and what
-// rounding it left (22 bits of f16, 16 of bf16), in a second pass over V.
+// PIECES: 16-bit numbers whose sum enters the value product for a probability: p rounded, then
+// what the rounding left, rounded again, and so on (launch_pieces has the rule).  Three bf16 hold
+// an f32 exactly, two hold 16 bits; two f16 hold 22 bits of 128 p, which the reference maximum keeps
+// below 2^15 and which keeps the second piece's error below 2^-32 of the row's sum.  One is the
+// ordinary form.  Bound like it by the LDS reads and matrix instructions, of which only the value
+// products are repeated: every V fragment is read once for all pieces (701 tokens, 32/8 heads of
+// 128: 1 piece 34 us, 2 39.8, 3 45.9; with V read again for the second piece 38.3; 4097 tokens
+// 2 pieces 219, 3 270, read again 221).
 // MULTI: the launch streams several KV blocks (segs.n > 1); otherwise block 0 only, whose
 // addresses the compiler keeps in registers for the whole kernel.
-template <typename T, int D, bool MULTI, bool FINE>
+template <typename T, int D, bool MULTI, int PIECES>
 __global__ __launch_bounds__(NTHREADS, 2) void attn_prefill_kernel(const AttnParams p,
                                                                    const KvSegs segs) {
   typedef Layout<D> L;
@@ -344,6 +351,8 @@ __global__ __launch_bounds__(NTHREADS, 2) void attn_prefill_kernel(const AttnPar
     for (int e = 0; e < 16; ++e) oacc[i][e] = 0.f;
   float m_run = -__builtin_inff();  // reference max of raw scores (q.k)
   float m_use = 0.f;                // m_run * c, or 0 while the row has seen nothing
+  // (a product and not part of the exponent, where it would cost small scores 7 bits)
+  constexpr float kPieceScale = PIECES > 1 && std::is_same<T, f16>::value ? 128.f : 1.f;
   float l_run = 0.f;                // this lane's partial row sum
 
   // mode: 1 every key of the tile visible to every row of the wave, 2 element-masked;
@@ -418,32 +427,26 @@ __global__ __launch_bounds__(NTHREADS, 2) void attn_prefill_kernel(const AttnPar
 #pragma unroll
         for (int e = 0; e < 16; ++e) oacc[dt][e] *= alpha;
     }
-    frag pf[4];
+    frag pf[PIECES][4];
     float pr[32];
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
         pr[kb * 16 + e] = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[kb][e], c, -m_use));
-        pf[kb * 2 + (e >> 3)][e & 7] = (T)pr[kb * 16 + e];
+        float rest = pr[kb * 16 + e] * kPieceScale;
+#pragma unroll
+        for (int pc = 0; pc < PIECES; ++pc) {
+          pf[pc][kb * 2 + (e >> 3)][e & 7] = (T)rest;
+          rest -= to_f32<T>(pf[pc][kb * 2 + (e >> 3)][e & 7]);
+        }
       }
-    // f32 row sum as a tree of independent adds (FINE still needs the probabilities)
-    if constexpr (FINE) {
-      float rs[16];
+    // f32 row sum as a tree of independent adds
 #pragma unroll
-      for (int e = 0; e < 16; ++e) rs[e] = pr[e] + pr[e + 16];
+    for (int w = 16; w >= 1; w >>= 1)
 #pragma unroll
-      for (int w = 8; w >= 1; w >>= 1)
-#pragma unroll
-        for (int e = 0; e < w; ++e) rs[e] += rs[e + w];
-      l_run += rs[0];
-    } else {
-#pragma unroll
-      for (int w = 16; w >= 1; w >>= 1)
-#pragma unroll
-        for (int e = 0; e < w; ++e) pr[e] += pr[e + w];
-      l_run += pr[0];
-    }
+      for (int e = 0; e < w; ++e) pr[e] += pr[e + w];
+    l_run += pr[0];
     // O^T += V^T . P^T: fragment of step s holds keys s*16 + {g*4..+3, 8+g*4..+3}
 #pragma unroll
     for (int dt = 0; dt < D / 32; ++dt) {
@@ -453,7 +456,9 @@ __global__ __launch_bounds__(NTHREADS, 2) void attn_prefill_kernel(const AttnPar
         vf[s] = read_tr_frag<frag>(sb + s * 16 * L::KROW + v_raddr[dt],
                                    sb + (s * 16 + 8) * L::KROW + v_raddr[dt]);
 #pragma unroll
-      for (int s = 0; s < 4; ++s) oacc[dt] = Mfma<T>::run(vf[s], pf[s], oacc[dt]);
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int pc = 0; pc < PIECES; ++pc) oacc[dt] = Mfma<T>::run(vf[s], pf[pc][s], oacc[dt]);
     }
     // the transposing reads of the next 16 columns overlap the products of these
     __builtin_amdgcn_sched_group_barrier(0x100, 8, 1);
@@ -461,23 +466,11 @@ __global__ __launch_bounds__(NTHREADS, 2) void attn_prefill_kernel(const AttnPar
     for (int j = 0; j < D / 32 - 1; ++j) {
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 1);
+        __builtin_amdgcn_sched_group_barrier(0x008, PIECES, 1);
         __builtin_amdgcn_sched_group_barrier(0x100, 2, 1);
       }
     }
-    __builtin_amdgcn_sched_group_barrier(0x008, 4, 1);
-    if constexpr (FINE) {
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int e = 0; e < 32; ++e) pf[e >> 3][e & 7] = (T)(pr[e] - to_f32<T>(pf[e >> 3][e & 7]));
-#pragma unroll
-      for (int dt = 0; dt < D / 32; ++dt)
-#pragma unroll
-        for (int s = 0; s < 4; ++s)
-          oacc[dt] = Mfma<T>::run(read_tr_frag<frag>(sb + s * 16 * L::KROW + v_raddr[dt],
-                                                     sb + (s * 16 + 8) * L::KROW + v_raddr[dt]),
-                                  pf[s], oacc[dt]);
-    }
+    __builtin_amdgcn_sched_group_barrier(0x008, 4 * PIECES, 1);
   };
 
   // ---- passes over the key block: list the tiles this workgroup needs, then stream them.
@@ -563,7 +556,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void attn_prefill_kernel(const AttnPar
   if (!row_ok) return;
   const float l_tot = sum_halves(l_run);
   const bool empty = !(l_tot > 0.f);
-  const float inv = empty ? 0.f : 1.f / l_tot;
+  const float inv = empty ? 0.f : 1.f / (l_tot * kPieceScale);
   const float lse_new = empty ? -__builtin_inff() : m_run * fabsf(scale) + logf(l_tot);
   // a key split's partial pair (offsets 0 without splits)
   const int64_t o_split = (int64_t)split * p.split_out;
@@ -639,7 +632,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void attn_prefill_kernel(const AttnPar
   }
 }
 
-template <typename T, int D, bool MULTI, bool FINE>
+template <typename T, int D, bool MULTI, int PIECES>
 int launch_typed(const AttnParams& params, const KvSegs& segs, hipStream_t st) {
   AttnParams p = params;
   const int hp = MULTI ? 1 : std::max(p.heads_per_wg, 1);
@@ -660,10 +653,10 @@ int launch_typed(const AttnParams& params, const KvSegs& segs, hipStream_t st) {
   const int64_t total = (int64_t)nqb * (p.Hq / hp) * p.B * (MULTI ? 1 : std::max(p.splits, 1));
   if (total == 0) return CEA_OK;
   CEA_REQUIRE(total < (int64_t)1 << 31, CEA_EUNSUPPORTED, "attention: grid too large");
-  const hipError_t e = reserve_lds<attn_prefill_kernel<T, D, MULTI, FINE>>(Layout<D>::LDS_BYTES);
+  const hipError_t e = reserve_lds<attn_prefill_kernel<T, D, MULTI, PIECES>>(Layout<D>::LDS_BYTES);
   CEA_REQUIRE(e == hipSuccess, CEA_ELAUNCH, "attention: cannot reserve %d bytes of LDS: %s",
               Layout<D>::LDS_BYTES, hipGetErrorString(e));
-  hipLaunchKernelGGL((attn_prefill_kernel<T, D, MULTI, FINE>), dim3((unsigned)total), dim3(NTHREADS),
+  hipLaunchKernelGGL((attn_prefill_kernel<T, D, MULTI, PIECES>), dim3((unsigned)total), dim3(NTHREADS),
                      Layout<D>::LDS_BYTES, st, p, segs);
   CEA_CHECK_LAUNCH("attention_prefill");
   return CEA_OK;
@@ -778,31 +771,40 @@ bool prefill_segs_supported(const AttnParams& p, const KvSegs& segs) {
   return tiles == p.ntiles && tiles < ((int64_t)1 << 24);
 }
 
-template <bool MULTI, bool FINE>
-static int launch_as(const AttnParams& p, const KvSegs& segs, hipStream_t st) {
+// Blocks whose position rows are 16-byte aligned take one piece.  The others (an odd number of
+// keys, an odd first slot) ran on the generic kernel, whose probabilities are f32, and keep that
+// with two pieces of f16 and three of bf16 (a 16-bit result is the f32 one rounded, so the count
+// does not look at it).  2-norm errors against 64 bits over 41 to 20001 keys, generic kernel /
+// here: f32 results bf16 8.1e-8 to 3.1e-5 / 6.5e-8 to 9.7e-7 (two pieces 6.6e-7 to 2.5e-6), f16
+// 8.0e-8 to 3.1e-5 / 6.7e-8 to 9.1e-7; bf16 results 1.45e-3 to 1.67e-3 on both, f16 1.79e-4 to
+// 2.10e-4 / 1.79e-4 to 2.09e-4 (2.9e-4 with one).  701 tokens of 32/8 heads take 9393 us on the
+// generic kernel.  The rule looks at the batch stride of a single row as well: an odd number of
+// keys decides, however many rows there are.
+static bool aligned_positions(const KvSegs& segs) {
+  for (int i = 0; i < segs.n; ++i)
+    if (segs.seg[i].kps_b % 2 || !al16(segs.seg[i].k_pos)) return false;
+  return true;
+}
+
+template <typename T, int D, bool MULTI>
+static int launch_pieces(const AttnParams& p, const KvSegs& segs, hipStream_t st) {
+  constexpr int kUnaligned = std::is_same<T, bf16>::value ? 3 : 2;
+  if (aligned_positions(segs)) return launch_typed<T, D, MULTI, 1>(p, segs, st);
+  return launch_typed<T, D, MULTI, kUnaligned>(p, segs, st);
+}
+
+template <bool MULTI>
+static int launch_dispatch(const AttnParams& p, const KvSegs& segs, hipStream_t st) {
   if (p.in_dtype == CEA_BF16) {
-    if (p.D == 128) return launch_typed<bf16, 128, MULTI, FINE>(p, segs, st);
-    if (p.D == 64) return launch_typed<bf16, 64, MULTI, FINE>(p, segs, st);
+    if (p.D == 128) return launch_pieces<bf16, 128, MULTI>(p, segs, st);
+    if (p.D == 64) return launch_pieces<bf16, 64, MULTI>(p, segs, st);
   } else if (p.in_dtype == CEA_F16) {
-    if (p.D == 128) return launch_typed<f16, 128, MULTI, FINE>(p, segs, st);
-    if (p.D == 64) return launch_typed<f16, 64, MULTI, FINE>(p, segs, st);
+    if (p.D == 128) return launch_pieces<f16, 128, MULTI>(p, segs, st);
+    if (p.D == 64) return launch_pieces<f16, 64, MULTI>(p, segs, st);
   }
   set_error("attention: MFMA path does not cover dtype %s, head size %d",
             dtype_name(p.in_dtype), p.D);
   return CEA_EUNSUPPORTED;
-}
-
-// Blocks whose position rows are not 16-byte aligned (an odd number of keys, an odd first slot)
-// used to run on the generic kernel, which keeps its probabilities in f32: they take the FINE
-// form, so their results are no further from exact than they were (f16, 701 tokens, 32/8 heads,
-// 2-norm: 2.00e-4 there and here, 2.9e-4 without the second pass; 9393 us there, 47 here, 34
-// without).
-template <bool MULTI>
-static int launch_dispatch(const AttnParams& p, const KvSegs& segs, hipStream_t st) {
-  bool fine = false;
-  for (int i = 0; i < segs.n; ++i)
-    fine = fine || segs.seg[i].kps_b % 2 || !al16(segs.seg[i].k_pos);
-  return fine ? launch_as<MULTI, true>(p, segs, st) : launch_as<MULTI, false>(p, segs, st);
 }
 
 int launch_attn_prefill_mfma(const AttnParams& p, hipStream_t st) {

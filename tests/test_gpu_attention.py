@@ -415,6 +415,43 @@ def test_key_positions_at_any_offset(cea, dev, rows, keys, first, d, dtype):
     assert err <= bound + 2 * score * v64.abs().max().item(), (err, bound, score)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("keys", [[33], [301], [129, 64, 107]], ids=str)
+def test_unaligned_positions_keep_f32_probabilities(cea, dev, keys, d, dtype):
+    """f32 results of blocks with an odd number of keys, alone and in a ring share, carry f32
+    probabilities.  Scores are below 1 here, so a probability's error is that of the f32
+    exponential and of its pieces (2^-23 and 2^-22 at most) and the sums add no more than about
+    as much; errors of the keys are independent, as their weights in the result are, so its
+    2-norm error relative to the result is bounded by the per-key error: 2^-21 is twice their sum.
+    Probabilities of 16 bits (two bf16 pieces) measure 1.4e-6 to 1.8e-6 here, and 3e-4 to 2e-3 as
+    one piece."""
+    n = sum(keys)
+    g = torch.Generator().manual_seed(n + d)
+    q = (0.1 * torch.randn(1, n, 4, d, generator=g)).to(dtype).to(dev)
+    k = torch.randn(1, n, 2, d, generator=g).to(dtype).to(dev)
+    v = torch.randn(1, n, 2, d, generator=g).to(dtype).to(dev)
+    pos = torch.arange(n).view(1, n).to(dev)
+    if len(keys) == 1:
+        out, lse = cea.attention_with_lse(q, k, v, pos, pos)
+    else:
+        group, start = cea.LocalGroup(len(keys), 0), 0
+        for r, m in enumerate(keys):
+            part = slice(start, start + m)
+            group.set_shard(r, k=k[:, part], v=v[:, part],
+                            pos=torch.arange(start, start + m, device=dev).view(1, m))
+            start += m
+        own = group.shard(0)
+        out, lse = cea.sequence_parallel.ring_attention_with_lse(
+            q, own["k"], own["v"], pos, own["pos"], group, keys)
+    torch.cuda.synchronize()
+    co, cl = ref.attention_with_lse(q.cpu().double(), k.cpu().double(), v.cpu().double(),
+                                    pos.cpu(), pos.cpu(), route="math")
+    err = (out.cpu().double() - co).norm() / co.norm()
+    assert err.item() <= 2.0 ** -21, err
+    assert (lse.cpu().double() - cl).abs().max().item() <= 2.0 ** -18
+
+
 @pytest.mark.parametrize("batch,queries,keys,hkv", [
     (1, 1, 1, 1),       # one key
     (1, 2, 65, 2),      # one key past a 64-key chunk
