@@ -452,6 +452,73 @@ def test_unaligned_positions_keep_f32_probabilities(cea, dev, keys, d, dtype):
     assert (lse.cpu().double() - cl).abs().max().item() <= 2.0 ** -18
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("rows,queries,keys", [
+    (2, 80, [131]),            # partial tiles, padding slots
+    (1, 301, [301]),           # several query blocks and tiles, some fully visible
+    (1, 300, [129, 64, 107]),  # a ring share: several blocks in one launch
+    (1, 20, [1101]),           # key splits
+], ids=str)
+def test_unaligned_positions_with_values_that_are_not_finite(cea, dev, rows, queries, keys, d, dtype):
+    """Blocks with an odd number of keys: NaN in the keys and values of hidden slots (padding, or
+    after the query) stays out of a row, +inf, -inf and NaN in the values of visible ones reach
+    it as in a sum, and nothing else changes."""
+    n = sum(keys)
+    g = torch.Generator().manual_seed(n + d)
+    q = torch.randn(rows, queries, 4, d, generator=g).to(dtype)
+    k = torch.randn(rows, n, 2, d, generator=g).to(dtype)
+    v = torch.randn(rows, n, 2, d, generator=g).to(dtype)
+    kp = torch.arange(n).repeat(rows, 1)
+    qp = torch.arange(n - queries, n).repeat(rows, 1)
+    kp[:, 5::17] = -1
+    inf = float("inf")
+    for key, feature, value in [(3, 0, inf), (n // 2, 1, -inf), (n // 2 + 1, 2, inf), (n // 2 + 2, 2, -inf),
+                                (n - 12, 7, float("nan")), (n - 2, 5, -inf), (n - 3, d - 1, inf)]:
+        kp[:, key] = key
+        v[:, key, key % 2, feature] = value
+    hidden = kp < 0
+    k[hidden] = float("nan")
+    v[hidden] = float("nan")
+    # the result with zeros in their place, and which of them a row sees
+    finite = torch.isfinite(v)
+    k0, v0 = torch.nan_to_num(k, nan=0.0), torch.where(finite, v, torch.zeros_like(v))
+    ro, rl = ref.attention_with_lse(q.double(), k0.double(), v0.double(), qp, kp, route="math")
+    vis = ((kp[:, None, :] >= 0) & (kp[:, None, :] <= qp[:, :, None])).double()
+    up = (torch.isnan(v) | (v == inf)) & ~hidden[:, :, None, None]
+    down = (torch.isnan(v) | (v == -inf)) & ~hidden[:, :, None, None]
+    for sign, plane in ((1, up), (-1, down)):
+        count = torch.matmul(vis, plane.double().flatten(2)).view(rows, queries, 2, d)
+        ro = ro + torch.where(count.repeat_interleave(2, 2) > 0, sign * inf, 0.0)
+
+    def check(out, what):
+        out = out.cpu().double()
+        assert torch.equal(torch.isnan(out), torch.isnan(ro)), what
+        assert torch.equal(torch.isinf(out), torch.isinf(ro)), what
+        assert torch.equal(out[torch.isinf(ro)], ro[torch.isinf(ro)]), what
+        ok = torch.isfinite(ro)
+        assert (out[ok] - ro[ok]).abs().max().item() <= 2e-2, what
+
+    q, k, v, qp = (t.to(dev) for t in (q, k, v, qp))
+    if len(keys) == 1:
+        out, lse = cea.attention_with_lse(q, k, v, qp, kp.to(dev))
+        plain = cea.attention.attention(q, k, v, qp, kp.to(dev))
+    else:
+        group, start = cea.LocalGroup(len(keys), 0), 0
+        for r, m in enumerate(keys):
+            pos = torch.empty(1, m, dtype=torch.int64, device=dev).copy_(kp[:, start:start + m])
+            group.set_shard(r, k=k[:, start:start + m], v=v[:, start:start + m], pos=pos)
+            start += m
+        own = group.shard(0)
+        out, lse = cea.sequence_parallel.ring_attention_with_lse(
+            q, own["k"], own["v"], qp, own["pos"], group, keys)
+        plain = cea.ring_attention(q, own["k"], own["v"], qp, own["pos"], group, keys)
+    torch.cuda.synchronize()
+    check(out, "f32")
+    check(plain, "16 bits")
+    assert (lse.cpu().double() - rl).abs().max().item() <= 1e-3
+
+
 @pytest.mark.parametrize("batch,queries,keys,hkv", [
     (1, 1, 1, 1),       # one key
     (1, 2, 65, 2),      # one key past a 64-key chunk
