@@ -898,6 +898,8 @@ static bool aligned_positions(const KvSegs& segs) {
   return true;
 }
 
+bool prefill_aligned_positions(const AttnParams& p) { return aligned_positions(single_segment(p)); }
+
 template <typename T, int D, bool MULTI>
 static int launch_pieces(const AttnParams& p, const KvSegs& segs, hipStream_t st) {
   constexpr int kUnaligned = std::is_same<T, bf16>::value ? 3 : 2;

@@ -336,6 +336,14 @@ static int run_prefill_split(const AttnParams& p, int S, char* ws, hipStream_t s
   return launch_merge(m, st);
 }
 
+// Whether the prefill kernel takes the call.  It needs the workspace for its tile summaries;
+// calls with unaligned position rows, which run on the generic kernel otherwise, are not refused
+// for a workspace too small for them.
+static bool use_prefill(const AttnParams& p, const char* ws, size_t ws_bytes) {
+  if (p.Sk == 0 || !prefill_mfma_supported(p)) return false;
+  return prefill_aligned_positions(p) || (ws != nullptr && ws_bytes >= tile_bytes(p.B, p.Sk));
+}
+
 // Runs one attention call with a prepared parameter block.  allow_decode = false keeps the
 // call off the split-KV decode kernels, whose workspace (chunk partials) is larger than the
 // tile summaries the other kernels need.
@@ -344,7 +352,7 @@ static int run_attention(AttnParams& p, char* ws, size_t ws_bytes, hipStream_t s
   if (allow_decode && p.Sk > 0 && use_decode(p))
     return run_decode(&p, 1, nullptr, nullptr, ws, ws_bytes, st);
   if (p.Sk > 0 && f32_mfma_supported(p)) return launch_attn_f32_mfma(p, st);
-  if (p.Sk > 0 && prefill_mfma_supported(p)) {
+  if (use_prefill(p, ws, ws_bytes)) {
     const size_t need = tile_bytes(p.B, p.Sk);
     CEA_REQUIRE(ws != nullptr && ws_bytes >= need, CEA_ENOSPACE,
                 "attention: workspace of %zu bytes needed, %zu given", need, ws_bytes);
@@ -492,7 +500,7 @@ int cea_attention_merge_final(const cea_tensor* q, const cea_tensor* k, const ce
   p.fs_s = final_out->stride[1];
   p.fs_h = final_out->stride[2];
   p.final_dtype = final_out->dtype;
-  if (p.Sk > 0 && !use_decode(p) && prefill_mfma_supported(p))
+  if (p.Sk > 0 && !use_decode(p) && use_prefill(p, (const char*)workspace, workspace_bytes))
     return run_attention(p, (char*)workspace, workspace_bytes, st);
   // other kernels: merge into the running pair, then cast it (a one-partial merge)
   p.final_out = nullptr;

@@ -209,6 +209,8 @@ int launch_tile_info_segs(const KvSegs& segs, int32_t B, TileInfo* tiles, int32_
 // the KV block of p as a one-entry segment table
 KvSegs single_segment(const AttnParams& p);
 bool prefill_mfma_supported(const AttnParams& p);
+// the block's position rows are 16-byte aligned (see attn_prefill.hip)
+bool prefill_aligned_positions(const AttnParams& p);
 // p carries q / out / lse / head map / row strides; the blocks come from segs (p.k, p.v,
 // p.k_pos and p.Sk are not read); p.ntiles and p.tiles cover all blocks
 bool prefill_segs_supported(const AttnParams& p, const KvSegs& segs);

@@ -90,3 +90,35 @@ def test_key_split_matches_oracle_and_unsplit(cea, dev, case):
     torch.cuda.synchronize()
     assert torch.equal(po, so) and torch.equal(pl, sl)
     assert plain.dtype == torch.bfloat16 and torch.equal(plain, so.to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("keys", [301, 300])
+def test_workspace_too_small_for_the_summaries(cea, dev, keys):
+    """An odd number of keys runs without a workspace as well (on the generic kernel), alone and
+    as the last merge of a ring; an even one is refused, as it always was."""
+    q, k, v, qp, kp = _inputs(1, 40, keys, 4, 2, 128, "aligned")
+    nat = cea._native
+    lib = nat.load_library()
+    t = [x.to(dev) for x in (q, k, v, qp, kp)]
+    args = [byref(nat.tensor_arg(x)) for x in t]
+    stream = nat.stream_of(dev)
+    ws = torch.empty(32, dtype=torch.uint8, device=dev)
+    ro, rl = ref.attention_with_lse(q, k, v, qp, kp)
+    for ptr, size in ((None, 0), (ws.data_ptr(), 32)):
+        out = torch.empty(1, 40, 4, 128, device=dev)
+        lse = torch.empty(1, 4, 40, device=dev)
+        o, l = nat.tensor_arg(out), nat.tensor_arg(lse)
+        rc = lib.cea_attention_with_lse(*args, 1, 128 ** -0.5, None, 0, byref(o), byref(l), 0, ptr, size, stream)
+        if keys % 2 == 0:
+            assert rc == -4, nat.last_error()
+            continue
+        assert rc == 0, nat.last_error()
+        run_o, run_l = torch.zeros_like(out), torch.full_like(lse, float("-inf"))
+        fin = torch.empty(1, 40, 4, 128, dtype=torch.bfloat16, device=dev)
+        rc = lib.cea_attention_merge_final(*args, 1, 128 ** -0.5, None, 0, byref(nat.tensor_arg(run_o)),
+                                           byref(nat.tensor_arg(run_l)), byref(nat.tensor_arg(fin)), ptr, size,
+                                           stream)
+        torch.cuda.synchronize()
+        assert rc == 0, nat.last_error()
+        assert_attention_close(out, lse, ro, rl, torch.bfloat16, "without a workspace")
+        assert torch.equal(fin, out.to(torch.bfloat16))
