@@ -501,6 +501,15 @@ bool mfma_path(const GemmParams& p, int dtype, int mode) {
   return true;
 }
 
+// f32 products of few terms each, bound by writing them: the matrix-core kernel, whose waves split
+// K, has waves without work there and adds their sums through LDS all the same.  Measured (us,
+// generic / matrix cores): 2048 x 2048 products of 16 11.7 / 25.1, of 64 19.2 / 25.4, of 96 25.8 /
+// 25.6; 512 x 2048 of 16 6.0 / 7.4, of 32 8.0 / 7.4; 8192 x 8192 of 64 203 / 356, of 128 356 / 367,
+// of 192 513 / 490.
+bool f32_output_bound(int64_t M, int64_t rows, int64_t K) {
+  return K <= 128 && M * rows >= (K <= 96 ? K << 16 : (int64_t)1 << 25);
+}
+
 template <typename T, int MODE, int ACT, int TB>
 int launch_tiles(GemmParams p, const TilePlan& pl, hipStream_t st) {
   typedef Tile<TB> L;
@@ -593,7 +602,9 @@ int launch_linear(const cea_tensor* x, const cea_tensor* wg, const cea_tensor* w
   const bool v16 = v8 && p.N % 8 == 0 && p.ldy % 8 == 0 && ((uintptr_t)p.y & 15) == 0;
   p.vec_out = v16 ? 2 : v8 ? 1 : 0;
   if (p.M == 0 || p.N == 0) return CEA_OK;
-  const bool mfma = mfma_path(p, x->dtype, mode);
+  bool mfma = mfma_path(p, x->dtype, mode);
+  if (x->dtype == CEA_F32 && f32_output_bound(p.M, (int64_t)p.N * (mode == kGated ? 2 : 1), p.K))
+    mfma = false;
   if (mfma && (p.M <= kSkinnyTokens || x->dtype == CEA_F32))
     return launch_linear_skinny(p, x->dtype, mode, act, st);
   switch (x->dtype) {

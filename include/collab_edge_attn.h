@@ -332,7 +332,8 @@ int cea_gated_mul(const cea_tensor* gate, const cea_tensor* up, cea_tensor* out,
  *   x [M, K], weight [N, K], bias [N] or NULL, y [M, N]: one dtype (bf16 / f16 / f32 / f64),
  *   innermost stride 1, any row strides (rows must not overlap); y must not overlap x, weight
  *   or bias.  bf16 / f16 (f32) with K and both row strides a multiple of 8 (4) and 16-byte
- *   aligned x and weight run on the matrix cores; everything else on a generic kernel.
+ *   aligned x and weight run on the matrix cores (f32 with K <= 128 only while the outputs are
+ *   few); everything else on a generic kernel.
  */
 int cea_linear(const cea_tensor* x, const cea_tensor* weight, const cea_tensor* bias,
                cea_tensor* y, void* stream);

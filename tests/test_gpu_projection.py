@@ -334,6 +334,8 @@ def test_linear_tile_heights_and_splits(cea, dev, dtype, m, k, n):
     (70, 36, 19),     # N not a multiple of 4, a K tail in the second slice
     (200, 132, 1030), # several token blocks in the grid
     (513, 516, 40),
+    (1030, 16, 600),  # bound by its outputs: the generic kernel
+    (1030, 96, 3050), # just too few outputs for it at this K
 ])
 def test_linear_f32_matrix_cores(cea, dev, m, k, n):
     """f32 operands on the matrix cores at ragged sizes, plain (every element within the f32
