@@ -248,11 +248,18 @@ __global__ __launch_bounds__(DTHREADS, 2) void decode_split_kernel(const P p) {
   const int key0 = (chunk - p.chunk_begin[part]) * p.chunk;
 
   // ---- visibility of the item's keys: thread t takes keys t, t + 256, ... of each chunk, so 16
-  // lanes hold one tile; every load is issued before the first wait (indices clamped)
+  // lanes hold one tile; every load is issued before the first wait (indices clamped).  A key no
+  // later than every query is seen by all of them and one later than every query by none, so the
+  // queries are gone through one by one only where a key of the wave lies between them (going
+  // through 16 of them for every key took 5 % of a call: 8 rows of 4096 keys, 32/4 heads of 64,
+  // 58.9 -> 56.4 us; 32 rows of 4096, 32/32 heads of 128, 349 -> 341).
   {
     constexpr int PER = CHMAX / DTHREADS;
     const int64_t* kp = p.k_pos[part] + b * p.kps[part][0];
     const int64_t kps = p.kps[part][1];
+    // (lane q holds query q's position: one load for all of them)
+    int64_t q_lane = 0;
+    if (p.Sq > 1) q_lane = p.q_pos[b * p.qps_b + (int64_t)min(lane, p.Sq - 1) * p.qps_s];
     int64_t pk[2][PER];
 #pragma unroll
     for (int ch = 0; ch < 2; ++ch)
@@ -262,19 +269,39 @@ __global__ __launch_bounds__(DTHREADS, 2) void decode_split_kernel(const P p) {
         if (ch < nch && u * DTHREADS < p.chunk)
           pk[ch][u] = kp[(int64_t)min(key0 + ch * p.chunk + u * DTHREADS + tid, Sk - 1) * kps];
       }
+    auto query = [&](int q) {
+      const uint32_t lo = __builtin_amdgcn_readlane((int)(uint32_t)q_lane, q);
+      return (int64_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(q_lane >> 32), q) << 32) | lo);
+    };
+    int64_t first = INT64_MAX, last = INT64_MAX;   // earliest and latest query
+    if (p.causal) {
+      first = last = p.q_pos[b * p.qps_b];
+#pragma unroll 1
+      for (int q = 1; q < p.Sq; ++q) first = min(first, query(q)), last = max(last, query(q));
+    }
+    const uint32_t all = (1u << p.Sq) - 1;
 #pragma unroll
     for (int ch = 0; ch < 2; ++ch) {
       uint64_t m = 0;
       if (ch < nch) {
         const int nkeys = min(p.chunk, Sk - key0 - ch * p.chunk);
         uint32_t words[PER] = {};
-        for (int q = 0; q < p.Sq; ++q) {
-          const int64_t qs = p.q_pos[b * p.qps_b + (int64_t)q * p.qps_s];
+        bool between = false;
 #pragma unroll
-          for (int u = 0; u < PER; ++u)
-            if (u * DTHREADS + tid < nkeys && pk[ch][u] >= 0 && (!p.causal || pk[ch][u] <= qs))
-              words[u] |= 1u << q;
+        for (int u = 0; u < PER; ++u) {
+          const bool key = u * DTHREADS + tid < nkeys && pk[ch][u] >= 0;
+          const bool seen = key && pk[ch][u] <= first;
+          words[u] = seen ? all : 0u;
+          between = between || (key && !seen && pk[ch][u] <= last);
         }
+        if (p.Sq > 1 && __ballot(between) != 0)
+#pragma unroll 1
+          for (int q = 0; q < p.Sq; ++q) {
+            const int64_t qs = query(q);
+#pragma unroll
+            for (int u = 0; u < PER; ++u)
+              if (u * DTHREADS + tid < nkeys && pk[ch][u] >= 0 && pk[ch][u] <= qs) words[u] |= 1u << q;
+          }
 #pragma unroll
         for (int u = 0; u < PER; ++u) {
           if (u * DTHREADS + tid < p.chunk) vis_s[ch * CHMAX + u * DTHREADS + tid] = (uint16_t)words[u];

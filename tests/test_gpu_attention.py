@@ -545,3 +545,23 @@ def test_decode_chunks(cea, dev, batch, queries, keys, hkv, d):
     ro, rl = ref.attention_with_lse(q, k, v, qp, kp, route="flash")
     torch.cuda.synchronize()
     assert_attention_close(out, lse, ro, rl, torch.bfloat16, f"decode {batch}x{queries}x{keys}")
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("queries", [2, 5, 16])
+def test_decode_of_several_tokens_visibility(cea, dev, queries, causal):
+    """Several query tokens in any order of positions, padding among them: keys before all of
+    them, after all of them and between them, in one chunk and over several, and padded slots."""
+    g = torch.Generator().manual_seed(queries)
+    for keys in (40, 700):
+        q = torch.randn(3, queries, 4, 64, generator=g).to(torch.bfloat16)
+        k = torch.randn(3, keys, 2, 64, generator=g).to(torch.bfloat16)
+        v = torch.randn(3, keys, 2, 64, generator=g).to(torch.bfloat16)
+        kp = torch.stack([torch.randperm(keys, generator=g) for _ in range(3)])
+        kp[:, ::7] = -1
+        qp = torch.randint(-1, keys, (3, queries), generator=g)
+        qp[0] = keys + torch.arange(queries)   # later than every key
+        out, lse = cea.attention_with_lse(*(t.to(dev) for t in (q, k, v, qp, kp)), causal=causal)
+        ro, rl = ref.attention_with_lse(q, k, v, qp, kp, causal=causal, route="flash")
+        torch.cuda.synchronize()
+        assert_attention_close(out, lse, ro, rl, torch.bfloat16, f"{queries} tokens, {keys} keys")
