@@ -835,23 +835,33 @@ bool decode_supported(int32_t Sq, int32_t Hq, int32_t Hkv, int32_t D, int32_t dt
   return Hq <= CEA_MAX_MAPPED_HEADS && decode_rows(Sq, 1) != 0;
 }
 
-// Work items a launch needs before its chunks grow past 256 keys: about two rounds of resident
-// workgroups (two per compute unit), since an item's start (positions, then its first tiles) is
-// hidden only behind the other resident item, and longer items have fewer of them.  Measured
-// (us, targets 8192 / 2048 / 1024; 32/8 heads, D = 128): 16 rows of 8000 keys 105 / 93 / 93, 32
-// of 4000 93 / 79 / 77, 8 of 32000 in two partitions 141 / 122 / 122.  An item's bytes per key
-// scale with the head size, so the count scales with it too (a head size of 64 takes half as
-// many, twice the keys each: the same bytes per item as at 128).
-static int64_t decode_item_target(int32_t D) { return (int64_t)1024 * D / 128; }
+// A number of items at D = 128, scaled with the head size as an item's bytes per key are (a head
+// size of 64 takes half as many, twice the keys each: the same bytes per item).
+static int64_t decode_items(int64_t n, int32_t D) { return n * D / 128; }
 
-int decode_plan_chunk(int64_t keys_per_head, int32_t B, int32_t units, int32_t D) {
-  // 64 keys (one tile per wave) up to 256 while the items are fewer than the compute units, so a
-  // short cache is read by all of them in one or two tiles each (one sequence of 300 keys, 8 KV
-  // heads: 12.3 us with 64-key chunks, 14.1 with 256); then 256..1024 by the item target
+// Keys per chunk.
+// * 64 (one tile per wave) up to 256 while the items are fewer than the compute units, so a short
+//   cache is read by all of them in one or two tiles each (one sequence of 300 keys, 8 KV heads:
+//   12.3 us with 64-key chunks, 14.1 with 256); but no more of them per row than the reduction
+//   reads ahead (one sequence of 8000 keys, 14/2 heads of 64: 125 chunks of 64 keys 19.7 us, 32
+//   of 256 12.9; 6000 keys 16.2 and 12.5).
+// * Then up to 1024 keys by a number of items (at D = 128).  1024 items are about two rounds of resident workgroups (two per compute unit): an
+//   item's start (positions, then its first tiles) is hidden only behind the other resident item,
+//   and longer items have fewer starts.  Measured (us, 8192 / 2048 / 1024 items; 32/8 heads, D =
+//   128): 16 rows of 8000 keys 105 / 93 / 93, 32 of 4000 93 / 79 / 77, 8 of 32000 in two
+//   partitions 141 / 122 / 122.
+// * 8192 for one token where even 1024-key chunks give 4096, 8 or more in a row: there the rounds are many and the last
+//   of them, with rows of uneven lengths, weighs more (us, 8192 / 1024 items: 32 rows of 8000 to
+//   16000 keys, 32/8 heads of 128 267 / 296, 16 of 2000 to 32000 189 / 209; with 8 tokens a row, whose
+//   items start with more work, 8 rows of 16000 to 32000 keys 301 / 260).
+int decode_plan_chunk(int64_t keys_per_head, int32_t B, int32_t units, int32_t Sq, int32_t D) {
   const int64_t heads = (int64_t)B * units;
+  auto chunks = [&](int ch) { return (keys_per_head + ch - 1) / ch; };
   int ch = 64;
-  while (ch < 256 && heads * ((keys_per_head + ch - 1) / ch) > 256) ch *= 2;
-  while (ch < CHMAX && heads * ((keys_per_head + ch - 1) / ch) > decode_item_target(D)) ch *= 2;
+  while (ch < 256 && (heads * chunks(ch) > 256 || chunks(ch) > RPF * RWAVES)) ch *= 2;
+  const bool many = Sq == 1 && chunks(CHMAX) >= 8 && heads * chunks(CHMAX) >= decode_items(4096, D);
+  const int64_t target = decode_items(many ? 8192 : 1024, D);
+  while (ch < CHMAX && heads * chunks(ch) > target) ch *= 2;
   return ch;
 }
 
@@ -862,14 +872,16 @@ int launch_attn_decode(const DecodeParams& params, hipStream_t st) {
   CEA_REQUIRE(p.chunk_begin[p.nparts] <= kDecodeMaxChunks, CEA_EUNSUPPORTED,
               "decode: %d chunks exceed %d", p.chunk_begin[p.nparts], kDecodeMaxChunks);
   // Pair items (half the partials written while K/V stream: those writes cost the read stream
-  // far more than their size) once chunks are at their largest and plentiful.  The last batch
+  // far more than their size) once chunks are at their largest and plentiful; three chunks stay
+  // single, for a pair takes twice the time of the third (32 rows of 3000 keys, 32/32 heads of
+  // 128: 217 us with pairs, 190 without).  The last batch
   // rows keep single chunks: enough of them for about two rounds of resident workgroups (two
   // per compute unit), so the launch ends on short workgroups.
   p.item_begin[0] = 0;
   for (int i = 0; i < p.nparts; ++i)
     p.item_begin[i + 1] = p.item_begin[i] + (p.chunk_begin[i + 1] - p.chunk_begin[i] + 1) / 2;
   const int64_t row_items = (int64_t)p.units * p.chunk_begin[p.nparts];
-  const bool pairs = p.chunk == CHMAX && p.B * row_items >= decode_item_target(p.D);
+  const bool pairs = p.chunk == CHMAX && p.chunk_begin[p.nparts] != 3 && p.B * row_items >= decode_items(1024, p.D);
   const int cus = device_cus();
   const int64_t tail_rows = row_items > 0 ? (4 * (int64_t)(cus > 0 ? cus : 256) + row_items - 1) / row_items : 1;
   p.pair_rows = pairs ? (int)max((int64_t)0, (int64_t)p.B - tail_rows) : 0;

@@ -234,6 +234,16 @@ def test_workspace_counts_decode_partials_only_for_the_decode_route(cea):
     assert lib.cea_attention_workspace_bytes(B, 1, Hq, Sk, Hkv, 64, 1) > tiles
 
 
+@pytest.mark.parametrize("keys", [4096, 6000, 8000, 12000, 16000])
+@pytest.mark.parametrize("Hq,Hkv,D,rows", [(14, 2, 64, 8), (16, 1, 128, 16)])
+def test_decode_of_one_sequence_keeps_few_chunks(cea, keys, Hq, Hkv, D, rows):
+    """One sequence with few KV heads takes chunks of fewer than 256 keys only while the row has
+    no more of them than the reduction reads ahead (48; its 256-key chunks may be more).  The
+    workspace is the partials alone: Hkv units x chunks x rows x (D + 2) floats."""
+    bytes_ = cea._native.load_library().cea_attention_workspace_bytes(1, 1, Hq, keys, Hkv, D, 1)
+    assert bytes_ <= Hkv * max(48, -(-keys // 256)) * rows * (D + 2) * 4 + 255
+
+
 def _split_plan(B, Sq, Hq, Sk, G):
     """Key splits of a bf16 prefill launch, restated from the rule the library documents:
     query heads per workgroup hp in {1, 2, 4, 8} (dividing G) with the fewest padded rows of
