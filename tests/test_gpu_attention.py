@@ -375,10 +375,10 @@ def test_decode_with_more_rows_per_kv_head_than_a_unit(cea, dev, shape):
 
 
 @pytest.mark.parametrize("shape", [
-    (2, 300, 8, 4),    # KV heads of all rows a multiple of 8: dealt to the XCDs in turn
-    (1, 520, 16, 8),   # the same, two query heads per KV head, a short last query block
-    (4, 258, 6, 3),    # query heads of all rows a multiple of 8 only
-    (1, 270, 6, 2),    # neither
+    (2, 300, 8, 4),    # one workgroup column (heads of a workgroup) on each XCD
+    (1, 520, 16, 8),   # the same, a short last query block
+    (4, 258, 6, 3),    # 12 columns: in the order of the grid
+    (1, 270, 6, 2),    # 2 columns: the same
 ], ids=str)
 def test_query_block_order(cea, dev, shape):
     """Every (row, head, query block) is computed once whichever way the blocks are dealt."""
@@ -389,6 +389,32 @@ def test_query_block_order(cea, dev, shape):
     ro, rl = ref.attention_with_lse(q, k, v, qp, kp, route="flash")
     torch.cuda.synchronize()
     assert_attention_close(out, lse, ro, rl, torch.bfloat16, str(case))
+
+
+@pytest.mark.parametrize("shape,kv_map", [
+    ((2, 512, 32, 8, 64), None),      # KV heads dealt in turn, 8 columns of 2 KV heads on each XCD
+    ((4, 300, 8, 4, 64), None),       # one column per KV head, 2 on each XCD, moving on by one
+    ((6, 700, 4, 4, 64), None),       # the same with 3, which stay in place
+    ((4, 512, 6, 3, 64), None),       # 24 columns, 12 KV heads: a run of columns on each XCD
+    ((2, 600, 8, 4, 64), [0, 1, 1, 2, 2, 2, 3, 3]),  # an irregular map, the same
+    ((3, 5000, 8, 8, 128), None),     # 3 KV heads of 2.6 MB on each XCD: a set of 2 and one of 1
+    ((3, 6000, 8, 8, 128), None),     # three sets of one
+], ids=str)
+def test_query_block_order_of_several_rows(cea, dev, shape, kv_map):
+    """Rows computed together and by fewer, where their blocks are dealt differently, have the same
+    bits: every (row, head, query block) is computed once.  (Alone, or two at a time where a row
+    alone would take key splits.)"""
+    B, S, Hq, Hkv, D = shape
+    g = torch.Generator(device=dev).manual_seed(S)
+    q, k, v = (torch.randn(B, S, h, D, generator=g, device=dev).to(torch.bfloat16) for h in (Hq, Hkv, Hkv))
+    pos = torch.arange(S, device=dev).repeat(B, 1)
+    pos[-1, S // 2:] = -1
+    out = cea.attention.attention(q, k, v, pos, pos, kv_map=kv_map)
+    n = 1 if S < 1024 else 2
+    for b in range(B - n + 1):
+        few = cea.attention.attention(*(t[b:b + n] for t in (q, k, v, pos, pos)), kv_map=kv_map)
+        assert torch.equal(out[b:b + n], few), b
+    torch.cuda.synchronize()
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
