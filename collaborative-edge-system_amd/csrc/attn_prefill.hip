@@ -182,10 +182,13 @@ __global__ __launch_bounds__(NTHREADS, 2) void attn_prefill_kernel(const AttnPar
   // one split and KV head (which read the same tiles) stay together as well.  A workgroup
   // holds hp query heads of one KV head's group (NWAVES / hp waves and BM / hp rows each), so
   // short query blocks do not leave most of its rows empty.
-  const int hp = MULTI ? 1 : max(p.heads_per_wg, 1);
-  const int rows_pb = BM / hp;  // query rows of one head in a workgroup
-  const int nqb = (p.Sq + rows_pb - 1) / rows_pb;
-  const int ngroups = p.Hq / hp;
+  // (a power of two, and the divisions by others are few and left out where they can be: each of
+  // them is some 40 instructions at the start of every workgroup)
+  const int hp_log2 = MULTI ? 0 : __builtin_ctz(max(p.heads_per_wg, 1));
+  const int hp = 1 << hp_log2;
+  const int rows_pb = BM >> hp_log2;  // query rows of one head in a workgroup
+  const int nqb = (p.Sq + rows_pb - 1) >> (__builtin_ctz(BM) - hp_log2);
+  const int ngroups = p.Hq >> hp_log2;
   const int units = ngroups * p.B;
   const int total = nqb * units;
   const int nsplit = MULTI ? 1 : max(p.splits, 1);
@@ -202,38 +205,46 @@ __global__ __launch_bounds__(NTHREADS, 2) void attn_prefill_kernel(const AttnPar
     b = bh / ngroups;
   } else {
     int unit;
-    if ((units & 7) == 0) {
+    if (nqb == 1) {
+      qb = 0;
+      unit = (units & 7) == 0 ? (blk & 7) * (units >> 3) + (blk >> 3) : blk;
+    } else if ((units & 7) == 0) {
       const int per_xcd = units >> 3, i = blk >> 3;
-      const int set = i / (p.order_units * nqb);   // query heads taken together
+      // query heads taken together
+      const int set = p.order_units == per_xcd ? 0 : i / (p.order_units * nqb);
       const int r = i - set * p.order_units * nqb;
       const int size = min(p.order_units, per_xcd - set * p.order_units);
       qb = r / size;
-      const int per_kv = p.map.group > 0 ? ngroups / p.Hkv : 1;
+      const int per_kv = p.order_per_kv;
       // (an XCD hands its blocks to its 4 shader engines in turn: with an even number of units and
       // units of other rows next to each other, each engine would get the same units, and with
       // them the same row lengths, every time; so the units move on by one every two query blocks:
       // four prompts of 1000 to 2000 tokens, 32/4 heads of 64, 124 us without, 104 with)
       const int turn = per_kv % 4 != 0 && size % 2 == 0 ? qb >> 1 : 0;
-      const int u = set * p.order_units + (r + turn) % size;
-      if (p.map.group > 0 && ((p.B * p.Hkv) & 7) == 0)
-        unit = ((blk & 7) + 8 * (u / per_kv)) * per_kv + u % per_kv;
-      else
+      int u = r - qb * size;
+      if (turn != 0) u = (u + turn) % size;
+      u += set * p.order_units;
+      if (p.map.group > 0 && ((p.B * p.Hkv) & 7) == 0) {
+        const int kv = per_kv == 1 ? u : u / per_kv;
+        unit = ((blk & 7) + 8 * kv) * per_kv + (u - kv * per_kv);
+      } else {
         unit = (blk & 7) * per_xcd + u;
+      }
     } else {
       qb = blk / units;
-      unit = blk % units;
+      unit = blk - qb * units;
     }
     qb = nqb - 1 - qb;
-    hg = unit % ngroups;
-    b = unit / ngroups;
+    b = p.B == 1 ? 0 : unit / ngroups;
+    hg = unit - b * ngroups;
   }
   // (in scalar registers: left to itself the compiler kept the merged paths' values in vector
   // registers and the tile loop lost 2 %)
   qb = uniform(qb), b = uniform(b), hg = uniform(hg), split = uniform(split);
-  const int waves_ph = NWAVES / hp;
-  const int h = hg * hp + wave / waves_ph;   // this wave's query head
-  const int kvh = p.map.kv_of(hg * hp);      // one KV head for the whole workgroup
-  const int qrow0 = qb * rows_pb + (wave % waves_ph) * 32;  // this wave's first query row
+  const int waves_log2 = __builtin_ctz(NWAVES) - hp_log2;   // waves of one head
+  const int h = hg * hp + (wave >> waves_log2);   // this wave's query head
+  const int kvh = p.map.kv_of(hg * hp);           // one KV head for the whole workgroup
+  const int qrow0 = qb * rows_pb + (wave & ((1 << waves_log2) - 1)) * 32;  // this wave's first query row
 
   const int row = qrow0 + r;
   const bool row_ok = row < p.Sq;
@@ -758,6 +769,7 @@ int launch_typed(const AttnParams& params, const KvSegs& segs, hipStream_t st) {
   // 3 MB 514 together, 430 one by one), in sets of even size
   const int64_t kv_bytes = std::max<int64_t>((int64_t)p.ntiles * BN * Layout<D>::KROW * 2, 1);
   const int64_t per_kv = p.map.group > 0 ? p.Hq / hp / p.Hkv : 1;
+  p.order_per_kv = (int)per_kv;
   const int64_t heads = std::max<int64_t>(((int64_t)p.B * (p.Hq / hp) + 8 * per_kv - 1) / (8 * per_kv), 1);
   const int64_t fit = std::max<int64_t>(((int64_t)5 << 20) / kv_bytes, 1);
   const int64_t sets = (heads + fit - 1) / fit;

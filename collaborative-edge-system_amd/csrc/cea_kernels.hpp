@@ -44,8 +44,8 @@ struct AttnParams {
   // with 1 / heads_per_wg of the workgroup's query rows
   int32_t heads_per_wg;
   // set by the prefill launcher: workgroup columns (query heads / heads_per_wg) an XCD works
-  // through together
-  int32_t order_units;
+  // through together, and those of one KV head
+  int32_t order_units, order_per_kv;
 };
 
 // KV blocks of one prefill launch, in the order their tiles are visited (a ring share's
