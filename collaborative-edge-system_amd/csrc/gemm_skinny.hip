@@ -182,7 +182,9 @@ int launch_shape(const GemmParams& p, hipStream_t st) {
 
 // Weight blocks per workgroup: the count with the least bytes through the busiest compute unit,
 // rounds of workgroups times (RB weight blocks + M / 16 token blocks), since every workgroup
-// reads all of x and a unit takes in about 57 B/ns however the loads are arranged.  Measured
+// reads all of x and a unit takes in at most about 57 B/ns however the loads are arranged (over
+// whole launches at 32 tokens, by the L2's read requests, 43 for 4096 x 14336, of which two thirds
+// are x, and 29 for gated 2 x 14336 x 4096, whose 448 workgroups run in 1.75 rounds).  Measured
 // (us, RB 1 / 2 / 4): 4096 x 14336, 32 tokens 28.7 / 35.7 / 50.6; 6144 x 4096, 16 tokens 15.6 /
 // 13.1 / 16.0; gated 2 x 4864 x 896, 20 tokens - / 10.3 / 7.3.
 template <int MODE> int weight_blocks(const GemmParams& p) {

@@ -358,7 +358,9 @@ int cea_linear_gated(const cea_tensor* x, const cea_tensor* w_gate, const cea_te
  * The same projections with scratch: a call whose output tiles are too few to fill the device
  * may split K over several workgroups, their f32 sums in `workspace` (16-byte aligned, at most
  * cea_linear_workspace_bytes() of the call's sizes, N the output columns, gated 0 / 1; contents
- * need no initialisation).  With less, or NULL, they run unsplit, as the calls above.
+ * need no initialisation).  With less they take the best launch whose sums fit, with fewer splits
+ * or other tiles, and with NULL they run unsplit, as the calls above; the order of the f32 sums,
+ * and with it the last bits of a result, depends on that size.
  */
 size_t cea_linear_workspace_bytes(int64_t M, int64_t N, int64_t K, int32_t dtype, int32_t gated);
 int cea_linear_ws(const cea_tensor* x, const cea_tensor* weight, const cea_tensor* bias,
