@@ -423,8 +423,9 @@ def test_query_block_order_of_several_rows(cea, dev, shape, kv_map):
 def test_key_positions_at_any_offset(cea, dev, rows, keys, first, d, dtype):
     """Odd key counts and blocks that begin at an odd slot of a larger position buffer (rows of
     8-byte aligned positions).  Their probabilities keep the bits that 16-bit rounding drops: the
-    f32 result is within 2^-16 (bf16: p as two 8-bit pieces) or 2^-20 (f16: two 11-bit pieces) of
-    the largest |v|, for every probability is within half an ulp of that and they sum to 1."""
+    f32 result is within 2^-16 (bf16, whose three pieces hold more) or 2^-20 (f16: two 11-bit
+    pieces) of the largest |v|, for every probability is within half an ulp of that and they sum
+    to 1.  (test_unaligned_positions_keep_f32_probabilities has the tighter bound.)"""
     case = Case(rows, 80, keys, 4, 2, d, "random", True, seed=rows + keys)
     q, k, v, qp, kp = (t.to(dev) for t in case.tensors(dtype))
     buf = torch.full((rows, first + keys), 0, dtype=torch.int64, device=dev)
